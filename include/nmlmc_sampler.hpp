@@ -129,7 +129,7 @@ struct SamplerPolicy {
 
     // inner_sampler::sample_inner (nested_sampler.hpp:131-161) over units
     // [u0, u1) of draw group `tag` (samples [i0, i1)).
-    template <bool F32>
+    template <bool F32, bool TEST>
     __device__ static void units(const Args& A, uint32_t m, const ItemState&, uint32_t tag, uint64_t u0,
                                  uint64_t u1, uint64_t i0, uint64_t i1, SegAcc& s) {
         static_assert(!F32, "sampler classes run in the FP64 form");

@@ -18,9 +18,10 @@
 //   P::spu                      inner samples per unit
 //   P::kTwoValued               final draws of levels > 0 give SegAcc::s1c too
 //   P::init_item(A, m, item)    outer draw, start value (init_inner_sampler)
-//   P::units<F32>(A, item_idx, item, tag, u0, u1, i0, i1, acc)
+//   P::units<F32, TEST>(A, item_idx, item, tag, u0, u1, i0, i1, acc)
 //                               accumulate units [u0, u1) of draw group
-//                               [i0, i1) (samples) of draw group `tag`
+//                               [i0, i1) (samples) of draw group `tag`; the
+//                               second moments (SegAcc::s2, smm) only with TEST
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

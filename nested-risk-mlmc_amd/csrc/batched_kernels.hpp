@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_test(typen
         const uint64_t cur = fine ? cur_f : cur_c, units = fine ? uf : uc;
         const uint64_t u0 = j * S, u1 = (u0 + S < units) ? u0 + S : units;
         SegAcc s;
-        P::template units<MIXED>(A, m, it, (fine ? TAG_FINE_TEST : TAG_COARSE_TEST) + r, u0, u1, 0, cur, s);
+        P::template units<MIXED, true>(A, m, it, (fine ? TAG_FINE_TEST : TAG_COARSE_TEST) + r, u0, u1, 0, cur, s);
         const uint32_t q = it.inst;
         if (!RECHECK) {
             acc.work(q, s.work);
@@ -485,11 +485,11 @@ __device__ __forceinline__ void outer_phi(const BatchedCommon& c, const ItemStat
 }
 
 // Sum of inner samples [i0, i1) of draw group `tag`, by one lane.
-template <class P, bool F32>
+template <class P, bool F32, bool TEST>
 __device__ __forceinline__ SegAcc lane_group(const typename P::Args& A, uint32_t m, const ItemState& it,
                                              uint32_t tag, uint64_t i0, uint64_t i1) {
     SegAcc s;
-    P::template units<F32>(A, m, it, tag, i0 / P::spu, (i1 + P::spu - 1) / P::spu, i0, i1, s);
+    P::template units<F32, TEST>(A, m, it, tag, i0 / P::spu, (i1 + P::spu - 1) / P::spu, i0, i1, s);
     return s;
 }
 
@@ -579,7 +579,7 @@ __global__ __launch_bounds__(256) void k_b_redo_split(typename P::Args A) {
             }
             SegAcc s;
             const uint64_t i0 = (uint64_t)g * sh.n;
-            P::template units<false>(A, m, it, TAG_FINAL, k, k + 1, i0, i0 + sh.n, s);
+            P::template units<false, false>(A, m, it, TAG_FINAL, k, k + 1, i0, i0 + sh.n, s);
             cur += s.s1;
         }
         if (cur_g != ~0u) atomicAdd(&gsum[cur_g], cur);
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(256) void k_b_redo_seq(typename P::Args A) {
             SegAcc sa;
             const uint64_t ub = i0 / P::spu, ue = (i1 + P::spu - 1) / P::spu;
             for (uint64_t u = ub + threadIdx.x; u < ue; u += blockDim.x)
-                P::template units<false>(A, m, it, tag, u, u + 1, i0, i1, sa);
+                P::template units<false, false>(A, m, it, tag, u, u + 1, i0, i1, sa);
             const double v = wave_sum(sa.s1);
             const double vc = P::kTwoValued ? wave_sum(sa.s1c) : 0.;
             if ((threadIdx.x & 63) == 0) {
@@ -675,8 +675,8 @@ __device__ __forceinline__ bool whole_final(const typename P::Args& A, uint32_t 
     const FinalShape sh = final_shape(c, it);
     bool near = false;
     if (c.ell > 0 && !c.ep.antithetic) {
-        const SegAcc a = lane_group<P, MIXED>(A, m, it, TAG_FINAL, 0, it.nf);
-        const SegAcc b = lane_group<P, MIXED>(A, m, it, TAG_FINAL_COARSE, 0, it.nc);
+        const SegAcc a = lane_group<P, MIXED, false>(A, m, it, TAG_FINAL, 0, it.nf);
+        const SegAcc b = lane_group<P, MIXED, false>(A, m, it, TAG_FINAL_COARSE, 0, it.nc);
         acc.work(it.inst, a.work + b.work + 2 * P::group_work(A, it));
         acc.st(it.inst, 4, a.nu + b.nu);
         acc.st(it.inst, 5, a.nn + b.nn);
@@ -689,7 +689,7 @@ __device__ __forceinline__ bool whole_final(const typename P::Args& A, uint32_t 
         const double coeff = (double)(1.f / (float)sh.groups);
         double s1_big = 0., sab_big = 0., phi_small = 0.;
         for (uint32_t g = 0; g < sh.groups; g++) {
-            const SegAcc a = lane_group<P, MIXED>(A, m, it, TAG_FINAL, (uint64_t)g * sh.n, (uint64_t)(g + 1) * sh.n);
+            const SegAcc a = lane_group<P, MIXED, false>(A, m, it, TAG_FINAL, (uint64_t)g * sh.n, (uint64_t)(g + 1) * sh.n);
             acc.work(it.inst, a.work + P::group_work(A, it));
             acc.st(it.inst, 4, a.nu);
             acc.st(it.inst, 5, a.nn);
@@ -794,7 +794,7 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_final(type
             const uint64_t ub = i0 / P::spu, ue = (i1 + P::spu - 1) / P::spu;
             const uint64_t u0 = ub + j * c.S, u1 = (u0 + c.S < ue) ? u0 + c.S : ue;
             const ItemState& it = c.items[m];
-            P::template units<MIXED>(A, m, it, fe.kind == 2 ? TAG_FINAL_COARSE : TAG_FINAL, u0, u1, i0, i1, s);
+            P::template units<MIXED, false>(A, m, it, fe.kind == 2 ? TAG_FINAL_COARSE : TAG_FINAL, u0, u1, i0, i1, s);
             acc.work(it.inst, s.work);
             acc.st(it.inst, 4, s.nu);
             acc.st(it.inst, 5, s.nn);
@@ -895,7 +895,7 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_fused(type
             acc.st(q, 3, (c.cf.max == c.cf.base));
         } else {
             acc.st(q, 0, c.cf.base);
-            const SegAcc t = lane_group<P, MIXED>(A, (uint32_t)m, it, TAG_FINE_TEST, 0, c.cf.base);
+            const SegAcc t = lane_group<P, MIXED, true>(A, (uint32_t)m, it, TAG_FINE_TEST, 0, c.cf.base);
             acc.work(q, t.work + P::group_work(A, it));
             acc.st(q, 4, t.nu);
             acc.st(q, 5, t.nn);
@@ -917,7 +917,7 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_fused(type
                 it.nc = c.cc.max;
             } else {
                 acc.st(q, 0, c.cc.base);
-                const SegAcc t = lane_group<P, MIXED>(A, (uint32_t)m, it, TAG_COARSE_TEST, 0, c.cc.base);
+                const SegAcc t = lane_group<P, MIXED, true>(A, (uint32_t)m, it, TAG_COARSE_TEST, 0, c.cc.base);
                 acc.work(q, t.work + P::group_work(A, it));
                 acc.st(q, 4, t.nu);
                 acc.st(q, 5, t.nn);

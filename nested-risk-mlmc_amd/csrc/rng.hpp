@@ -169,31 +169,58 @@ __device__ __forceinline__ void boxmuller_f64(uint64_t u0, uint64_t u1, double& 
     y = c * r;
 }
 
+// The same pair through the device library's functions; it differs from the
+// one above by a last-place rounding in some of its values.  The model's batched FP64
+// form keeps it: its difference sums are, at the levels where no outer sample
+// straddles the threshold, nothing but rounding residues of means that are
+// equal, and with other roundings they are other residues.
+__device__ __forceinline__ void boxmuller_f64_lib(uint64_t u0, uint64_t u1, double& x, double& y) {
+    double s, c;
+    sincos(3.1415926535897932 * uneg11_f64(u0), &s, &c);
+    const double r = sqrt(-2. * log(u01_f64(u1)));
+    x = s * r;
+    y = c * r;
+}
+
 // FP32 Box-Muller for the mixed form: the same words, u1 -> (0,1] in float and
-// u0 -> [-1,1], sin/cos(pi x) and log in hardware-accelerated single precision.
-// The float of u1 carries a relative error up to 2^-24, i.e. an absolute error
-// of about 2^-24 in ln u1; the radius r = sqrt(-2 ln u1) then has an error of
+// u0 -> [-1,1], sin/cos(pi x) and log by the hardware's instructions, as the
+// polar parts of the pair (r sn, r cs) and r2 = r^2.
+//
+// The angle goes in revolutions, which is what the instructions take: u0 2^-65
+// from its high word, off by at most 2^-33 (an angle error below 2^-30).  The
+// float of u1 carries a relative error of about 2^-24, i.e. an absolute error
+// of that in ln u1; the radius r = sqrt(-2 ln u1) then has an error of
 // about 2^-24 / r, which for u1 near 1 (small r) would reach 100% (a word of
 // u1 >= 2^64 - 2^39 rounds to 1: radius 0 against an FP64 radius up to 2^-12).
 // Words with u1 > 1 - 2^-8 (top byte all ones, 2^-8 of them) therefore take
 // the radius from q = 1 - u01(u1) = ~u1 2^-64 + 2^-65, whose float is accurate
 // to 2^-24 relative: -ln(1 - q) = q (1 + q/2 + q^2/3 + q^3/4), truncation below
-// 2^-33 relative for q <= 2^-8.  Elsewhere r >= 2^-3.5 and the error stays
-// below about 2^-20.5.
-__device__ __forceinline__ void boxmuller_f32(uint64_t u0, uint64_t u1, float& x, float& y) {
-    const float a = (float)(int64_t)u0 * 0x1p-63f + 0x1p-64f;
-    float s, c;
-    __sincosf(3.14159265358979f * a, &s, &c);
-    float r2;
-    if ((uint32_t)(u1 >> 32) < 0xFF000000u) {
-        r2 = -2.f * __logf((float)u1 * 0x1p-64f + 0x1p-65f);
-    } else {
-        const float q = (float)(~u1) * 0x1p-64f + 0x1p-65f;
+// 2^-33 relative for q <= 2^-8.  Elsewhere r >= 2^-3.5 and the normals stay
+// within 2^-20.5 (2^-19 for u1 below 2^-20, which 2^-20 of the words have).
+//
+// Bound by VALU issue, as the Threefry block before it.  Whole-word conversions
+// (a shift, clamp and scaling each), the C functions' denormal steps and the
+// correctly rounded root took 85 slots of 64 lanes after a block of 116; this
+// way 11, with an error no larger anywhere in 2^20 pairs (edges included): at
+// most 2^-20.5 against 2^-19.8, rms 2^-23.3 against 2^-22.9.
+__device__ __forceinline__ void bm_polar_f32(uint64_t u0, uint64_t u1, float& sn, float& cs, float& r, float& r2) {
+    const float h = (float)(int32_t)(u0 >> 32) * 0x1p-32f;
+    sn = __builtin_amdgcn_sinf(h);
+    cs = __builtin_amdgcn_cosf(h);
+    const uint32_t hi = (uint32_t)(u1 >> 32), lo = (uint32_t)u1;
+    const float u = __builtin_fmaf((float)hi, 0x1p-32f, __builtin_fmaf((float)lo, 0x1p-64f, 0x1p-65f));
+    r2 = __builtin_amdgcn_logf(u) * -0x1.62e43p+0f;  // log2 u times -2 ln 2
+    if (hi >= 0xFF000000u) {  // one wave in five meets such a lane
+        const float q = __builtin_fmaf((float)~hi, 0x1p-32f, __builtin_fmaf((float)~lo, 0x1p-64f, 0x1p-65f));
         r2 = 2.f * q * (1.f + q * (0.5f + q * (0x1.555556p-2f + q * 0.25f)));
     }
-    const float r = __fsqrt_rn(r2);
-    x = s * r;
-    y = c * r;
+    r = __builtin_amdgcn_sqrtf(r2);
+}
+__device__ __forceinline__ void boxmuller_f32(uint64_t u0, uint64_t u1, float& x, float& y) {
+    float sn, cs, r, r2;
+    bm_polar_f32(u0, u1, sn, cs, r, r2);
+    x = sn * r;
+    y = cs * r;
 }
 
 // Word q of the stream keyed {k0, k1}.
