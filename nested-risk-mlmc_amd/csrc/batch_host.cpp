@@ -157,16 +157,17 @@ int Engine::batch_sample(uint32_t ell, const uint64_t* Ms, sample_output* outs) 
         if ((e = hipHostMalloc(&h_btab, 8 * tab_off[nc])) != hipSuccess) return hip_fail(e, "hipHostMalloc batch tables");
         btab_cap = tab_off[nc];
     }
-    if (nc * n > inst_out_cap) {
+    const size_t per = (size_t)kInstReps * n;  // records a chunk
+    if (nc * per > inst_out_cap) {
         if (d_inst_out) hipFree(d_inst_out);
         if (h_inst_out) hipHostFree(h_inst_out);
         d_inst_out = h_inst_out = nullptr;
         inst_out_cap = 0;
-        if ((e = hipMalloc(&d_inst_out, sizeof(Partial) * nc * n)) != hipSuccess)
+        if ((e = hipMalloc(&d_inst_out, sizeof(Partial) * nc * per)) != hipSuccess)
             return hip_fail(e, "hipMalloc batch accumulators");
-        if ((e = hipHostMalloc(&h_inst_out, sizeof(Partial) * nc * n)) != hipSuccess)
+        if ((e = hipHostMalloc(&h_inst_out, sizeof(Partial) * nc * per)) != hipSuccess)
             return hip_fail(e, "hipHostMalloc batch accumulators");
-        inst_out_cap = nc * n;
+        inst_out_cap = nc * per;
     }
     std::vector<PortfolioBatchTables> tabs(nc);
     for (size_t k = 0; k < nc; k++) {
@@ -227,7 +228,7 @@ int Engine::batch_sample(uint32_t ell, const uint64_t* Ms, sample_output* outs) 
         const uint64_t Mk = ((const uint64_t*)h_btab)[tab_off[k] + tabs[k].n_seg];
         H.c.M = Mk;
         H.c.offset = 0;
-        H.c.inst_out = d_inst_out + k * n;
+        H.c.inst_out = d_inst_out + k * per;
         H.bt = tabs[k];
         const Shape sh = batched_shape(ell, Mk, 1, H.c, 0);
         H.c.S = sh.S;
@@ -255,13 +256,13 @@ int Engine::batch_sample(uint32_t ell, const uint64_t* Ms, sample_output* outs) 
         hipEventElapsedTime(&ms, ev0, ev1);
         ms_total += ms;
     }
-    if (nc && (e = hipMemcpy(h_inst_out, d_inst_out, sizeof(Partial) * nc * n, hipMemcpyDeviceToHost)) != hipSuccess)
+    if (nc && (e = hipMemcpy(h_inst_out, d_inst_out, sizeof(Partial) * nc * per, hipMemcpyDeviceToHost)) != hipSuccess)
         return hip_fail(e, "hipMemcpy batch accumulators");
     uint64_t reev = 0, flips = 0, rck = 0;
     for (uint32_t i = 0; i < n; i++) {
         Partial t;
         std::memset(&t, 0, sizeof(t));
-        for (size_t k = 0; k < nc; k++) {
+        for (size_t k = 0; k < nc * kInstReps; k++) {
             const Partial& a = h_inst_out[k * n + i];
             for (int j = 0; j < kMaxPhi * kMaxMoments; j++) {
                 t.f[j] += a.f[j];

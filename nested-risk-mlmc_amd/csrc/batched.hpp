@@ -73,19 +73,37 @@ struct FinalEntry {
     uint32_t item, group, done, kind;  // kind: 0 antithetic / fine-only, 1 plain fine, 2 plain coarse
 };
 
+// Atomics on one 128-byte line are performed one after another, 11.4 ns each
+// (side by side on different lines), whichever block or XCD they come from: a
+// counter that 10^5 waves bump takes over a millisecond.  So a block's level
+// sums go to one of kAccReps records (its blockIdx modulo kAccReps; the host
+// adds the records up), queue appends are gathered per wave and per block
+// (Appends), and counters used in the same phase lie on lines of their own.
+// With one record and one append a wave iteration, the first pass of the
+// adaptive model's level 0 (8.4M outer samples, 7% refining) took 1.60 ms, all of it
+// its appends; gathered, 1.20 ms, and the first refinement round 122 us (238).
+constexpr uint32_t kAccReps = 32;
+constexpr uint32_t kInstReps = 8;  // a batch's per-instance records: one set per XCD
+struct alignas(128) AccRecord {
+    Partial p;
+};
+
 // Device control block of one level call.
 struct BatchedCtl {
-    uint32_t cnt_f[kMaxRounds + 1], cnt_c[kMaxRounds + 1];
-    uint32_t n_whole;  // outer samples whose final fits one segment (one lane, no atomics)
+    AccRecord acc[kAccReps];  // level sums, work and stats (atomics)
+    alignas(128) uint32_t cnt_f[kMaxRounds + 1];
+    alignas(128) uint32_t cnt_c[kMaxRounds + 1];
+    alignas(128) uint32_t n_pend;  // fused first pass: outer samples left for the final phase
+    // mixed: decisions of round r left to the FP64 recheck
+    alignas(128) uint32_t rc_f[kMaxRounds + 1];
+    alignas(128) uint32_t rc_c[kMaxRounds + 1];
+    alignas(128) uint32_t nreeval;  // outer samples listed for the split FP64 redo (reeval[0 ..])
+    alignas(128) uint32_t nreeval_seq;  // outer samples listed for the sequential redo (reeval[M - 1 ..] downwards)
+    alignas(128) uint32_t n_whole;  // outer samples whose final fits one segment (one lane, no atomics)
     uint32_t class_cnt[kMaxClasses], class_off[kMaxClasses + 1], class_cur[kMaxClasses];
     uint32_t final_total;
-    uint32_t nreeval;      // outer samples listed for the split FP64 redo (reeval[0 ..])
-    uint32_t nreeval_seq;  // outer samples listed for the sequential redo (reeval[M - 1 ..] downwards)
     uint32_t overflow;
-    uint32_t n_pend;  // fused first pass: outer samples left for the final phase
     uint32_t count_done;  // blocks of k_b_final_count that have counted
-    uint32_t rc_f[kMaxRounds + 1], rc_c[kMaxRounds + 1];  // mixed: decisions of round r left to the FP64 recheck
-    Partial acc;  // level sums, work and stats (atomics)
 };
 
 // Per-lane accumulation of one segment.
@@ -287,6 +305,82 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool want) {
     return base + (uint32_t)__popcll(mask & below);
 }
 
+// Queue appends of a block of 256 threads, gathered in LDS: each wave collects
+// the item ids its lanes append to queue q (compacted, one LDS slot an id), and
+// hands them on when more than 64 are there (one atomic on the queue's counter
+// for all of them) or, at the kernel's end, together with the block's other
+// waves (one atomic a block and queue).  counter(q) gives the queue's counter,
+// write(q, id, slot) stores id into the queue's slot.
+template <int Q>
+struct Appends {
+    static constexpr uint32_t kCap = 128;
+    struct Store {
+        uint32_t n[4][Q];
+        uint32_t base[Q];
+        uint32_t id[4][Q][kCap];
+    };
+    __device__ __forceinline__ static Store& store() {
+        __shared__ Store s;
+        return s;
+    }
+    // LDS accesses of one wave are performed in order: this keeps the
+    // compiler's order the written one.
+    __device__ __forceinline__ static void wave_fence() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __device__ __forceinline__ void init() {
+        const uint32_t lane = threadIdx.x & 63;
+        if (lane < (uint32_t)Q) store().n[threadIdx.x >> 6][lane] = 0;
+        wave_fence();
+    }
+    // The wave's active lanes call it together.
+    template <class C, class W>
+    __device__ __forceinline__ void add(int q, bool want, uint32_t id, const C& counter, const W& write) {
+        const uint64_t mask = __ballot(want);
+        if (!mask) return;
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
+        uint32_t* const ids = store().id[wave][q];
+        const uint32_t have = store().n[wave][q];
+        uint32_t now = have + (uint32_t)__popcll(mask);
+        wave_fence();
+        if (want) ids[have + (uint32_t)__popcll(mask & below)] = id;
+        wave_fence();
+        if (now > kCap - 64) {
+            const uint64_t active = __ballot(1);
+            const uint32_t first = (uint32_t)__ffsll((long long)active) - 1;
+            uint32_t base = 0;
+            if (lane == first) base = atomicAdd(counter(q), now);
+            base = __shfl(base, (int)first, 64);
+            const uint32_t nact = (uint32_t)__popcll(active);
+            for (uint32_t i = (uint32_t)__popcll(active & below); i < now; i += nact) write(q, ids[i], base + i);
+            now = 0;
+        }
+        store().n[wave][q] = now;  // the same value from every active lane
+        wave_fence();
+    }
+    // All threads of the block call it, after their last add.
+    template <class C, class W>
+    __device__ __forceinline__ void finish(const C& counter, const W& write) {
+        Store& s = store();
+        __syncthreads();
+        if (threadIdx.x < (uint32_t)Q) {
+            const uint32_t q = threadIdx.x;
+            const uint32_t total = s.n[0][q] + s.n[1][q] + s.n[2][q] + s.n[3][q];
+            s.base[q] = total ? atomicAdd(counter((int)q), total) : 0;
+        }
+        __syncthreads();
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            uint32_t off = s.base[q];
+            for (uint32_t w = 0; w < wave; w++) off += s.n[w][q];
+            for (uint32_t i = lane; i < s.n[wave][q]; i += 64) write(q, s.id[wave][q][i], off + i);
+        }
+    }
+};
+
 // Fields shared by every problem's batched arguments (P::Args embeds it as .c).
 struct BatchedCommon {
     EngineParams ep;
@@ -313,7 +407,7 @@ struct BatchedCommon {
     double* redo_acc;    // [kRedoSlots x kRedoGroups] FP64 group sums of the redo
     uint32_t* redo_cnt;  // [kRedoSlots] parts of the redo done
     BatchedCtl* ctl;
-    Partial* inst_out;   // batch of problems: per-instance level accumulators (else NULL: ctl->acc)
+    Partial* inst_out;   // batch of problems: level accumulators [kInstReps x n_inst] (else NULL: ctl->acc)
     uint32_t n_inst;     // instances in the batch (0 for a single problem)
     uint32_t zero_ctl;   // 1: the chain starts by clearing ctl (and inst_out); 0: ctl is clear already
     uint32_t xcd_sliced; // 1: grid-stride passes split per XCD (xcd_range)
@@ -326,10 +420,10 @@ struct BatchedCommon {
 
 // Level accumulators of a block, behind one interface for the two layouts:
 //   MULTI = false (one problem): LaneAcc registers and the lanes' LDS moment
-//     columns, flushed into c.ctl->acc;
+//     columns, flushed into one of c.ctl->acc;
 //   MULTI = true (a batch of problems; every outer sample carries its
 //     instance): per-instance sums in LDS, added with LDS atomics and flushed
-//     into c.inst_out[instance].
+//     into one set of c.inst_out.
 // MOM: the kernel finishes outer samples (moment sums are kept).  init and
 // flush must be reached by every thread of the block.
 constexpr uint32_t kMaxInst = 64;
@@ -393,25 +487,27 @@ struct BlockAcc {
     template <bool MOM>
     __device__ __forceinline__ void flush(const BatchedCommon& c) {
         if (!MULTI) {
-            block_flush<MOM>(r, &c.ctl->acc);
+            block_flush<MOM>(r, &c.ctl->acc[blockIdx.x % kAccReps].p);
             return;
         }
         __syncthreads();
+        Partial* const mine = c.inst_out + (blockIdx.x % kInstReps) * c.n_inst;
         for (uint32_t i = threadIdx.x; i < c.n_inst * kInstD; i += blockDim.x) {
             const double v = inst_sums()[i];
             const uint32_t q = i / kInstD, f = i - q * kInstD;
-            Partial* out = &c.inst_out[q];
+            Partial* out = &mine[q];
             if (v != 0.) atomicAdd(f < kMaxMoments ? &out->f[f] : (f < 2 * kMaxMoments ? &out->d[f - kMaxMoments] : &out->work), v);
         }
         for (uint32_t i = threadIdx.x; i < c.n_inst * kStatsExt; i += blockDim.x) {
             const unsigned long long v = inst_stats()[i];
-            if (v) atomicAdd((unsigned long long*)&c.inst_out[i / kStatsExt].stats[i % kStatsExt], v);
+            if (v) atomicAdd((unsigned long long*)&mine[i / kStatsExt].stats[i % kStatsExt], v);
         }
     }
 };
 
 // Defined once (reduce.hip): clears the control block (and a batch's
-// per-instance accumulators).
+// kInstReps sets of n_inst accumulators).
+constexpr uint32_t kZeroBlocks = 4;
 __global__ void k_b_zero(BatchedCtl* ctl, Partial* inst_out, uint32_t n_inst);
 // Launches k_b_zero on the control block alone.
 hipError_t launch_clear_ctl(BatchedCtl* ctl, hipStream_t s);

@@ -210,6 +210,15 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_test(typen
     acc.template init<false>(c);
     TestEntry* const lf = RECHECK ? c.rq[0] : c.tf[r & 1];
     TestEntry* const lc_ = RECHECK ? c.rq[1] : c.tc[r & 1];
+    // Refined outer samples go to round r + 1 at doubled count (queues 0 and 1,
+    // fine and coarse), mixed decisions in doubt to round r's recheck (2, 3).
+    Appends<MIXED ? 4 : 2> app;
+    app.init();
+    auto counter = [&](int q) { return q == 0 ? &c.ctl->cnt_f[r + 1] : q == 1 ? &c.ctl->cnt_c[r + 1] : q == 2 ? &c.ctl->rc_f[r] : &c.ctl->rc_c[r]; };
+    auto write = [&](int q, uint32_t m, uint32_t slot) {
+        TestEntry* const dst = q == 0 ? c.tf[(r + 1) & 1] : q == 1 ? c.tc[(r + 1) & 1] : c.rq[q - 2];
+        dst[slot] = TestEntry{0., 0., 0., 0., m, 0};
+    };
     const XcdRange xr = xcd_range(total, c.xcd_sliced);
     for (uint64_t k = xr.k0; k < xr.end; k += xr.stride) {
         const bool fine = k < segs_f;
@@ -283,19 +292,14 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_test(typen
                 }
             }
         }
-        // Refined outer samples go to round r + 1 at doubled count.
-        const uint32_t sf = wave_append(&c.ctl->cnt_f[r + 1], append && fine);
-        const uint32_t sc = wave_append(&c.ctl->cnt_c[r + 1], append && !fine);
-        if (append) {
-            if (fine) c.tf[(r + 1) & 1][sf] = TestEntry{0., 0., 0., 0., m, 0};
-            else c.tc[(r + 1) & 1][sc] = TestEntry{0., 0., 0., 0., m, 0};
-        }
-        if (MIXED) {
-            const uint32_t rf = wave_append(&c.ctl->rc_f[r], recheck && fine);
-            const uint32_t rc = wave_append(&c.ctl->rc_c[r], recheck && !fine);
-            if (recheck) c.rq[fine ? 0 : 1][fine ? rf : rc] = TestEntry{0., 0., 0., 0., m, 0};
+        app.add(0, append && fine, m, counter, write);
+        app.add(1, append && !fine, m, counter, write);
+        if constexpr (MIXED) {
+            app.add(2, recheck && fine, m, counter, write);
+            app.add(3, recheck && !fine, m, counter, write);
         }
     }
+    app.finish(counter, write);
     acc.template flush<false>(c);
 }
 
@@ -498,7 +502,8 @@ __device__ __forceinline__ SegAcc lane_group(const typename P::Args& A, uint32_t
 // to the level accumulator with atomics.
 __device__ __forceinline__ void redo_finish(const BatchedCommon& c, uint64_t m, const ItemState& it, double phi_f,
                                          double phi_c) {
-    Partial* out = c.inst_out ? &c.inst_out[it.inst] : &c.ctl->acc;
+    Partial* out = c.inst_out ? &c.inst_out[(blockIdx.x % kInstReps) * c.n_inst + it.inst]
+                              : &c.ctl->acc[blockIdx.x % kAccReps].p;
     double p = 1.;
     for (uint32_t j = 0; j < c.ep.fine_moments; j++) {
         p *= phi_f;
@@ -721,7 +726,8 @@ __device__ __forceinline__ void list_reeval(const BatchedCommon& c, bool reeval,
     if (split) {
         c.reeval[slot] = m;
         if (slot < kRedoSlots) {
-            for (uint32_t g = 0; g < kRedoGroups; g++) astore(&c.redo_acc[(uint64_t)slot * kRedoGroups + g], 0.);
+            const uint32_t groups = final_shape(c, c.items[m]).groups;
+            for (uint32_t g = 0; g < groups; g++) astore(&c.redo_acc[(uint64_t)slot * kRedoGroups + g], 0.);
             __hip_atomic_exchange(&c.redo_cnt[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     } else if (reeval) {
@@ -881,6 +887,19 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_fused(type
     acc.template init<true>(c);
     const bool test_f = c.cf.max > 2 * c.cf.base;
     const bool test_c = c.ell > 0 && c.cc.max > 2 * c.cc.base;
+    // Queues: 0, 1 round 1's fine and coarse tests; 2 the final phase's outer
+    // samples; 3, 4 round 0's rechecks.
+    Appends<MIXED ? 5 : 3> app;
+    app.init();
+    auto counter = [&](int q) { return q == 0 ? &c.ctl->cnt_f[1] : q == 1 ? &c.ctl->cnt_c[1] : q == 2 ? &c.ctl->n_pend : q == 3 ? &c.ctl->rc_f[0] : &c.ctl->rc_c[0]; };
+    auto write = [&](int q, uint32_t m, uint32_t slot) {
+        if (q == 2) {
+            c.pend[slot] = m;
+            return;
+        }
+        TestEntry* const dst = q == 0 ? c.tf[1] : q == 1 ? c.tc[1] : c.rq[q - 3];
+        dst[slot] = TestEntry{0., 0., 0., 0., m, 0};
+    };
     const XcdRange xr = xcd_range(c.M, c.xcd_sliced);
     for (uint64_t m = xr.k0; m < xr.end; m += xr.stride) {
         ItemState it;
@@ -961,20 +980,16 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_fused(type
                 w.phi32_c = it.phi32_c;
             }
         }
-        const uint32_t sf = wave_append(&c.ctl->cnt_f[1], app_f);
-        const uint32_t sc = wave_append(&c.ctl->cnt_c[1], app_c);
-        const uint32_t sp = wave_append(&c.ctl->n_pend, pending);
-        if (app_f) c.tf[1][sf] = TestEntry{0., 0., 0., 0., (uint32_t)m, 0};
-        if (app_c) c.tc[1][sc] = TestEntry{0., 0., 0., 0., (uint32_t)m, 0};
-        if (pending) c.pend[sp] = (uint32_t)m;
-        if (MIXED) {
+        app.add(0, app_f, (uint32_t)m, counter, write);
+        app.add(1, app_c, (uint32_t)m, counter, write);
+        app.add(2, pending, (uint32_t)m, counter, write);
+        if constexpr (MIXED) {
             list_reeval<P>(c, reeval, (uint32_t)m);
-            const uint32_t rf = wave_append(&c.ctl->rc_f[0], rck_f);
-            const uint32_t rc = wave_append(&c.ctl->rc_c[0], rck_c);
-            if (rck_f) c.rq[0][rf] = TestEntry{0., 0., 0., 0., (uint32_t)m, 0};
-            if (rck_c) c.rq[1][rc] = TestEntry{0., 0., 0., 0., (uint32_t)m, 0};
+            app.add(3, rck_f, (uint32_t)m, counter, write);
+            app.add(4, rck_c, (uint32_t)m, counter, write);
         }
     }
+    app.finish(counter, write);
     acc.template flush<true>(c);
 }
 
@@ -996,7 +1011,7 @@ hipError_t launch_batched_level(const typename P::Args& A0, uint32_t blocks, hip
     typename P::Args A = A0;
     A.c.fused = fused_applies<P>(A.c) ? 1u : 0u;
     const bool rule1 = A.c.ep.adapt_rule == 1;
-    if (A.c.zero_ctl) hipLaunchKernelGGL(k_b_zero, dim3(1), dim3(256), 0, s, A.c.ctl, A.c.inst_out, A.c.n_inst);
+    if (A.c.zero_ctl) hipLaunchKernelGGL(k_b_zero, dim3(kZeroBlocks), dim3(256), 0, s, A.c.ctl, A.c.inst_out, A.c.n_inst);
     hipError_t e = P::launch_outer(A, s);
     if (e != hipSuccess) return e;
     // Mixed form: the FP64 recheck of round r's uncertain decisions, before

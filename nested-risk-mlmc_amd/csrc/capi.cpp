@@ -505,6 +505,19 @@ int Engine::batched_common(uint32_t ell, uint64_t M, uint64_t outer_offset, Batc
     return prepare_batched(std::min(M, batched_chunk()), c);
 }
 
+// Adds a control block's kAccReps records of level sums to t.
+static void add_records(const BatchedCtl& b, Partial& t) {
+    for (uint32_t k = 0; k < kAccReps; k++) {
+        const Partial& a = b.acc[k].p;
+        for (int j = 0; j < kMaxPhi * kMaxMoments; j++) {
+            t.f[j] += a.f[j];
+            t.d[j] += a.d[j];
+        }
+        t.work += a.work;
+        for (int j = 0; j < kStatsExt; j++) t.stats[j] += a.stats[j];
+    }
+}
+
 int Engine::run_batched(uint32_t ell, uint64_t M, BatchedCommon& c, sample_output* out,
                         const std::function<hipError_t()>& launch, double* tr_phi_f, double* tr_phi_c,
                         uint64_t* tr_nf, uint64_t* tr_nc) {
@@ -583,13 +596,7 @@ int Engine::run_batched(uint32_t ell, uint64_t M, BatchedCommon& c, sample_outpu
         float ms = 0;
         hipEventElapsedTime(&ms, ev0, ev1);
         ms_total += ms;
-        const Partial& a = bat_ctl_h->acc;
-        for (int i = 0; i < 16; i++) {
-            total.f[i] += a.f[i];
-            total.d[i] += a.d[i];
-        }
-        total.work += a.work;
-        for (int i = 0; i < kStatsExt; i++) total.stats[i] += a.stats[i];
+        add_records(*bat_ctl_h, total);
     }
     c.offset = offset0;
     last_ms = ms_total;
@@ -735,12 +742,7 @@ int Engine::sample_levels(uint32_t n, const uint32_t* ells, const uint64_t* Ms, 
         const BatchedCtl& b = sweep_slots[k];
         Partial& t = tot[sweep_chain_level[k]];
         if (b.overflow) redo[sweep_chain_level[k]] = 1;
-        for (int j = 0; j < kMaxPhi * kMaxMoments; j++) {
-            t.f[j] += b.acc.f[j];
-            t.d[j] += b.acc.d[j];
-        }
-        t.work += b.acc.work;
-        for (int j = 0; j < kStatsExt; j++) t.stats[j] += b.acc.stats[j];
+        add_records(b, t);
     }
     uint64_t reev = 0, flips = 0, rck = 0;
     for (uint32_t i = 0; i < n; i++) {

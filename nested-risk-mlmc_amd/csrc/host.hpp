@@ -168,7 +168,7 @@ struct Engine {
     void* d_btab = nullptr;                  // per-chunk segment tables (grown)
     void* h_btab = nullptr;                  // pinned staging of the same
     size_t btab_cap = 0;
-    Partial* d_inst_out = nullptr;           // [chunks x n] per-instance accumulators (grown)
+    Partial* d_inst_out = nullptr;           // [chunks x kInstReps x n] per-instance accumulators (grown)
     Partial* h_inst_out = nullptr;           // pinned
     size_t inst_out_cap = 0;
     int batch_begin(uint32_t n);

@@ -84,17 +84,18 @@ hipError_t launch_reduce_partials(const Partial* P, uint32_t n, Partial* out, hi
 }
 
 hipError_t launch_clear_ctl(BatchedCtl* ctl, hipStream_t s) {
-    hipLaunchKernelGGL(k_b_zero, dim3(1), dim3(256), 0, s, ctl, (Partial*)nullptr, 0u);
+    hipLaunchKernelGGL(k_b_zero, dim3(kZeroBlocks), dim3(256), 0, s, ctl, (Partial*)nullptr, 0u);
     return hipGetLastError();
 }
 
 __global__ void k_b_zero(BatchedCtl* ctl, Partial* inst_out, uint32_t n_inst) {
-    uint32_t* p = (uint32_t*)ctl;
-    const uint32_t n = sizeof(BatchedCtl) / 4;
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-    uint32_t* q = (uint32_t*)inst_out;
-    const uint32_t nq = inst_out ? n_inst * (uint32_t)(sizeof(Partial) / 4) : 0;
-    for (uint32_t i = threadIdx.x; i < nq; i += blockDim.x) q[i] = 0;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    uint64_t* p = (uint64_t*)ctl;
+    const uint32_t n = sizeof(BatchedCtl) / 8;
+    for (uint32_t i = t; i < n; i += stride) p[i] = 0;
+    uint64_t* q = (uint64_t*)inst_out;
+    const uint32_t nq = inst_out ? kInstReps * n_inst * (uint32_t)(sizeof(Partial) / 8) : 0;
+    for (uint32_t i = t; i < nq; i += stride) q[i] = 0;
 }
 
 }  // namespace nmlmc
