@@ -44,6 +44,22 @@ struct MixStock {
     float pad[2];
 };
 
+// One Exact option for the FP64 inner term (40 of an OptionRec's 64 bytes).
+struct ExactRec {
+    double K;        // strike
+    double Tt, sTt;  // T - tau and its root
+    double discp;    // w e^{-rT} / p; p = prob / prob_norm (sub-sampling 1), 1 / P (-1), 1 (0)
+    uint32_t stype;  // stock index << 8 | (type + 2)
+    uint32_t pad;
+};
+static_assert(sizeof(ExactRec) == 40, "Exact option record must stay 40 bytes");
+
+// Per-stock constants of the FP64 inner term: sigma, r - sigma^2 / 2 and that times
+// tau, sqrt(tau), S0, 1 / S0.
+struct ExactStock {
+    double sig, dcoef, ctau, stau, S0, invS0;
+};
+
 constexpr uint32_t kGuideLo = 0x7fffffffu, kGuideMulti = 0x80000000u;
 // Unbiased levels whose weight beta^(-e L) / (1 - beta^e) is tabulated.
 constexpr uint32_t kUnbLevels = 32;
@@ -62,6 +78,10 @@ struct PortfolioDevice {
     // the inner loss with the stock's parameters and the weight 1/p folded in.
     const MixRec* mix;
     const MixStock* mix_stocks;
+    // Exact options (method 1) in staged order: the FP64 constants of the
+    // inner term, the sub-sampling weight folded in.
+    const ExactRec* exact;
+    const ExactStock* exact_stocks;
     double w_est_const;  // the common W_est of all options, or -1 when they differ
     uint32_t nopt[3];
     const StockRec* stocks;

@@ -188,8 +188,9 @@ struct PortfolioPolicyT {
                 lvw &= lvw - 1;
                 st.init(seed, k1, ((uint64_t)tag << 40) | (w0 + j), 0, 0., 0);
                 uint32_t method;
-                prob = pick_option(pf, st, st, method, idx);
+                pick_option(pf, st, st, method, idx);
                 const OptionRec o = pf.options[2][idx];
+                prob = option_prob(pf, o);
                 unbiased_begin(pf, o, R, st, st, work, p);
                 // simulate_dt_d's step sizes
                 const double t = o.maturity - pf.tau;
@@ -309,24 +310,27 @@ struct PortfolioPolicyT {
             return;
         }
         if constexpr (EXACT_ONLY) {
+            s.nu += 2 * (u1 - u0);
+            s.nn += 2 * (u1 - u0);
             for (uint64_t u = u0; u < u1; u++) {
                 // FP64 (the FP32 loop returned above).  The sample's words: 0 method
                 // uniform (only method 1 has options), 1 option uniform (block 0),
                 // 2 and 3 the Box-Muller pair (block 1).
                 const uint64_t cu = ((uint64_t)tag << 40) | u;
                 const u64x2 blk0 = threefry2x64_20(0, cu, seed, k1);
-                const u64x2 blk1 = threefry2x64_20(1, cu, seed, k1);
                 const uint32_t idx = pick_cdf(pf, 1, u01_f64(blk0.a) * pf.compute_prob[1]);
-                s.nu += 2;
-                s.nn += 2;
-                const OptionRec o = pf.options[1][idx];
-                const double prob = o.prob / pf.prob_norm;
-                work += o.W_est;
-                double z0, z1, w64 = 0.;
+                // The record and the stock level are on their way while the
+                // second block and its normals are computed.
+                const ExactRec q = pf.exact[idx];
+                const double Rq = R[q.stype >> 8];
+                const u64x2 blk1 = threefry2x64_20(1, cu, seed, k1);
+                double z0, z1;
                 boxmuller_f64(blk1.a, blk1.b, z0, z1);
-                const double v = inner_exact_d(pf, o, R, z0, z1, w64) / prob;
+                work += pf.w_est_const >= 0. ? pf.w_est_const : pf.options[1][idx].W_est;
+                const double v = inner_exact_d(q, pf.exact_stocks[q.stype >> 8], pf.use_antithetic_risk,
+                                               pf.use_delta_cv, Rq, z0, z1);
                 a1 += v;
-                a2 += v * v;
+                if (TEST) a2 += v * v;
             }
         } else if (pf.subsample != 0) {
             // Inner samples by cost.  An Unbiased sample runs 8 * 4^L Milstein
@@ -362,7 +366,7 @@ struct PortfolioPolicyT {
                     DStream st;
                     st.init(seed, k1, ((uint64_t)tag << 40) | (w0 + j), 0, 0., 0);
                     uint32_t method, idx;
-                    const double prob = pick_option(pf, st, st, method, idx);
+                    pick_option(pf, st, st, method, idx);
                     if (method == 2 && pf.coupled) {
                         lv0 |= 1ull << j;  // a pass of their own, below
                         continue;
@@ -375,7 +379,6 @@ struct PortfolioPolicyT {
                         else lvw |= bit;
                         continue;
                     }
-                    const OptionRec o = pf.options[method][idx];
                     // Mixed form: the Exact terms in FP32, except in books with
                     // Unbiased options, whose FP64 paths dominate the work: there
                     // FP32 Exact terms save little and their error bound sends more
@@ -385,6 +388,7 @@ struct PortfolioPolicyT {
                         st.nn += 2;
                         float x, y, mag;
                         boxmuller_f32(second, first, x, y);
+                        const OptionRec o = pf.options[1][idx];
                         work += o.W_est;
                         float d;
                         if (pf.subsample == 1) {
@@ -396,7 +400,7 @@ struct PortfolioPolicyT {
                                                 (float)R[si], x, y, mag);
                         } else {
                             bool exact64;
-                            const float ip = (float)(1. / prob);
+                            const float ip = (float)pf.options_count;
                             d = inner_exact_f(pf, o, (float)R[o.stock_ind], x, y, mag, exact64) * ip;
                             mag *= ip;
                             redo64 |= exact64;
@@ -406,11 +410,12 @@ struct PortfolioPolicyT {
                         bab.add(mag);
                         mm += mag * (fabsf(d) + 0x1p-19f * mag);
                     } else if (method == 0) {
-                        add64(inner_bs_d(pf, o, R, work) / prob);
+                        const OptionRec o = pf.options[0][idx];
+                        add64(inner_bs_d(pf, o, R, work) / option_prob(pf, o));
                     } else {
                         const double z0 = st.randn();
                         const double z1 = st.randn();
-                        add64(inner_exact_d(pf, o, R, z0, z1, work) / prob);
+                        add64(exact_term(pf, idx, R, z0, z1, work));
                     }
                     s.nu += st.nu;
                     s.nn += st.nn;
@@ -425,17 +430,18 @@ struct PortfolioPolicyT {
                         DStream st;
                         st.init(seed, k1, ((uint64_t)tag << 40) | (w0 + j), 0, 0., 0);
                         uint32_t method, idx;
-                        const double prob = pick_option(pf, st, st, method, idx);
+                        pick_option(pf, st, st, method, idx);
+                        const OptionRec o = pf.options[2][idx];
+                        const double prob = option_prob(pf, o);
                         if (pf.coupled) {
                             double vc;
-                            const double vf =
-                                inner_coupled_d(pf, pf.options[2][idx], R, st, n_cpl, cs, two, work, vc) / prob;
+                            const double vf = inner_coupled_d(pf, o, R, st, n_cpl, cs, two, work, vc) / prob;
                             vc /= prob;
                             add64(vf);
                             dc += vc - vf;
                             ab += fabs(vc - vf);
                         } else {
-                            add64(inner_unbiased_d(pf, pf.options[2][idx], R, st, st, work) / prob);
+                            add64(inner_unbiased_d(pf, o, R, st, st, work) / prob);
                         }
                         s.nu += st.nu;
                         s.nn += st.nn;

@@ -184,34 +184,48 @@ int Engine::stage_portfolio(const portfolio_data* data) {
     P.coupled = (level_coupled && data->options[2].size) ? 1u : 0u;
     if (P.coupled && data->subsample != 1)
         return set_error(NMLMC_ERR_ARG, "level-coupled paths need sub-sampling mode 1");
-    // FP32 records of the Exact options and of the stocks for the mixed form.
+    // Records of the Exact options and of the stocks for the mixed (FP32) and the
+    // FP64 inner terms, in one upload.
     {
         const option_params* ex = (const option_params*)data->options[1].data;
         const size_t n1 = data->options[1].size;
-        std::vector<MixRec> mix(n1);
+        auto at = [](size_t off) { return (off + 63) & ~(size_t)63; };
+        const size_t o_ext = at(sizeof(MixRec) * n1), o_ms = at(o_ext + sizeof(ExactRec) * n1),
+                     o_es = at(o_ms + sizeof(MixStock) * d), size = o_es + sizeof(ExactStock) * d;
+        std::vector<char> tab(size, 0);
+        MixRec* mix = (MixRec*)tab.data();
+        ExactRec* ext = (ExactRec*)(tab.data() + o_ext);
+        MixStock* ms = (MixStock*)(tab.data() + o_ms);
+        ExactStock* es = (ExactStock*)(tab.data() + o_es);
         for (size_t j = 0; j < n1; j++) {
             const option_params& o = ex[j];
-            MixRec& q = mix[j];
-            q.K = (float)o.strike;
-            q.sTt = (float)std::sqrt(o.maturity - data->tau);
-            q.discp = (float)(o.w * std::exp(-data->r * o.maturity) * P.prob_norm / o.prob);
-            q.stype = (o.stock_ind << 8) | (uint32_t)(o.type + 2);
+            const double w = o.w * std::exp(-data->r * o.maturity);
+            const double Tt = o.maturity - data->tau, sTt = std::sqrt(Tt);
+            const uint32_t stype = (o.stock_ind << 8) | (uint32_t)(o.type + 2);
+            mix[j] = MixRec{(float)o.strike, (float)sTt, (float)(w * P.prob_norm / o.prob), stype};
+            const double discp = data->subsample == 1    ? w / (o.prob / P.prob_norm)
+                                 : data->subsample == -1 ? w * P.options_count
+                                                         : w;
+            ext[j] = ExactRec{o.strike, Tt, sTt, discp, stype, 0};
         }
-        if ((rc = upload(*this, mix.data(), n1, &P.mix))) return rc;
-        std::vector<MixStock> ms(d);
         for (uint32_t i = 0; i < d; i++) {
             const stock_params& st = stocks[i];
             const double dcoef = data->r - 0.5 * st.sigma * st.sigma;
             MixStock& q = ms[i];
-            std::memset(&q, 0, sizeof(q));
             q.sig = (float)st.sigma;
             q.dcoef = (float)dcoef;
             q.sigtau = (float)(st.sigma * std::sqrt(data->tau));
             q.S0e = (float)(st.S0 * std::exp(dcoef * data->tau));
             q.S0 = (float)st.S0;
             q.invS0 = (float)(1. / st.S0);
+            es[i] = ExactStock{st.sigma, dcoef, dcoef * data->tau, P.stau, st.S0, 1. / st.S0};
         }
-        if ((rc = upload(*this, ms.data(), d, &P.mix_stocks))) return rc;
+        const char* dev;
+        if ((rc = upload(*this, (const char*)tab.data(), size, &dev))) return rc;
+        P.mix = (const MixRec*)dev;
+        P.exact = (const ExactRec*)(dev + o_ext);
+        P.mix_stocks = (const MixStock*)(dev + o_ms);
+        P.exact_stocks = (const ExactStock*)(dev + o_es);
     }
     P.w_est_const = -1.;
     {

@@ -78,20 +78,10 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
         double s1 = 0., s2 = 0., work = 0.;
         for (uint64_t k = tid; k < count; k += 64 * W) {
             const uint64_t q = si.P + 3 * k;
-            const double u = u01_f64(stream_word(A.seed, k1, q));
-            uint32_t idx;
-            double prob;
-            if (pf.subsample == -1) {
-                idx = (uint32_t)(ceil(u * (double)pf.nopt[1]) - 1);
-                prob = 1. / pf.options_count;
-            } else {
-                idx = pick_cdf(pf, 1, u * pf.compute_prob[1]);
-                prob = pf.options[1][idx].prob / pf.prob_norm;
-            }
-            const OptionRec o = pf.options[1][idx];
+            const uint32_t idx = pick_in_method(pf, 1, u01_f64(stream_word(A.seed, k1, q)));
             double x, y;
             stream_bm_f64(A.seed, k1, q + 1, x, y);
-            const double v = inner_exact_d(pf, o, R, x, y, work) / prob;
+            const double v = exact_term(pf, idx, R, x, y, work);
             s1 += v;
             s2 += v * v;
         }
@@ -127,27 +117,17 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
             const uint64_t nvalid = count - c0 < 64 ? count - c0 : 64;
             const uint64_t q = si.P + base + (valid ? lane + 2 * __popcll(exact & below) : 0);
             if (valid) {
-                const double u = u01_f64(stream_word(A.seed, k1, q));
-                uint32_t idx;
-                double prob;
-                if (pf.subsample == -1) {
-                    idx = (uint32_t)(ceil(u * (double)pf.nopt[method]) - 1);
-                    prob = 1. / pf.options_count;
-                } else {
-                    idx = pick_cdf(pf, method, u * pf.compute_prob[method]);
-                    prob = pf.options[method][idx].prob / pf.prob_norm;
-                }
-                const OptionRec o = pf.options[method][idx];
+                const uint32_t idx = pick_in_method(pf, method, u01_f64(stream_word(A.seed, k1, q)));
                 double v;
                 if (method == 1) {
                     double x, y;
                     stream_bm_f64(A.seed, k1, q + 1, x, y);
-                    v = inner_exact_d(pf, o, R, x, y, work);
+                    v = exact_term(pf, idx, R, x, y, work);
                     nn += 2;
                 } else {
-                    v = inner_bs_d(pf, o, R, work);
+                    const OptionRec o = pf.options[0][idx];
+                    v = inner_bs_d(pf, o, R, work) / option_prob(pf, o);
                 }
-                v = v / prob;
                 s1 += v;
                 s2 += v * v;
             }
@@ -174,10 +154,10 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
                 // pick_option and the Exact branch of inner_sample_d: the
                 // method uniform is drawn, and method 1 is the only one.
                 uint32_t method, idx;
-                const double prob = pick_option(pf, sy, in, method, idx);
+                pick_option(pf, sy, in, method, idx);
                 const double z0 = in.randn();
                 const double z1 = in.randn();
-                d = inner_exact_d(pf, pf.options[1][idx], R, z0, z1, work) / prob;
+                d = exact_term(pf, idx, R, z0, z1, work);
             } else {
                 d = inner_sample_d<KIND != PAR_NO_UNBIASED>(pf, R, sy, in, work);
             }
