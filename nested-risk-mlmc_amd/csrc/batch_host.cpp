@@ -61,6 +61,9 @@ int Engine::batch_stage(uint32_t i, const portfolio_data* data, uint64_t s, cons
     for (void* p : b.allocs) hipFree(p);
     b.allocs.clear();
     b.allocs.swap(pf_allocs);
+    b.allocs.push_back(pf_blob);
+    pf_blob = nullptr;
+    pf_blob_cap = 0;
     b.pf = pf;
     b.bs_work = pf_bs_work;
     b.seed = s;

@@ -178,20 +178,25 @@ int Engine::ensure_ws(size_t n) {
 }
 
 // init_samplers (nested_sampler.hpp:618-644): both streams of thread t keyed
-// {seed, t} at position 0 (the OpenMP seeding, 640-641).
+// {seed, t} at position 0 (the OpenMP seeding, 640-641).  The states' memory and
+// the plain form's workspaces are kept from seeding to seeding (allocating and
+// freeing them cost a plain evaluation more than its smallest level call) and
+// released by init_nestedmc_sampler and cleanup_nestedmc_sampler.
 int Engine::seed_samplers(uint64_t s) {
     seed = s;
     int rc = ensure_device();
     if (rc) return rc;
-    free_samplers();
-    hipError_t e = hipMalloc(&d_states, sizeof(StreamState) * 2 * (size_t)cores);
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc states");
+    hipError_t e;
+    if (!d_states || states_cores != cores) {
+        free_samplers();
+        if ((e = hipMalloc(&d_states, sizeof(StreamState) * 2 * (size_t)cores)) != hipSuccess)
+            return hip_fail(e, "hipMalloc states");
+        states_cores = cores;
+    }
     e = hipMemsetAsync(d_states, 0, sizeof(StreamState) * 2 * (size_t)cores, stream);
     if (e != hipSuccess) return hip_fail(e, "hipMemset states");
     next_outer.assign(64, 0);
     tuned.clear();
-    e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
     return NMLMC_OK;
 }
 
@@ -969,6 +974,7 @@ void cleanup_nestedmc_sampler(void) {
     g_engine.free_batch();
     g_engine.free_samplers();
     g_engine.free_portfolio();
+    g_engine.free_stage();
     g_engine.free_batched();
     g_engine.inited = false;
     g_engine.problem = -1;

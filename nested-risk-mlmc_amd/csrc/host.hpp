@@ -43,11 +43,19 @@ struct Engine {
     uint32_t pf_phi_size = 1;
     double pf_bs_work = 0.;        // work of one init_inner_sampler call
     std::vector<void*> pf_allocs;
+    void* pf_blob = nullptr;       // the tables' block (stage_portfolio)
+    size_t pf_blob_cap = 0;
+    void* h_stage = nullptr;       // pinned: what staging uploads
+    size_t h_stage_cap = 0;
+    hipEvent_t stage_ev = nullptr; // its last upload is done
+    int stage_buffer(size_t size);
+    void free_stage();
     double* pf_R = nullptr;        // batched: outer states [M x d]
     float* pf_R32 = nullptr;       // their FP32 copies (same buffer, after the FP64 rows)
     size_t pf_R_cap = 0;
 
-    StreamState* d_states = nullptr;  // [2 cores]: parity streams (sync, inner)
+    StreamState* d_states = nullptr;  // [2 states_cores]: parity streams (sync, inner)
+    uint32_t states_cores = 0;
     Partial* d_partials = nullptr;    // [cores] or [batched groups]
     size_t partial_cap = 0;
     Partial* d_out = nullptr;         // the reduced record, then kReduceBlocks staging records

@@ -60,6 +60,7 @@ struct ExactStock {
     double sig, dcoef, ctau, stau, S0, invS0;
 };
 
+constexpr uint32_t kBlobChol = 256;
 constexpr uint32_t kGuideLo = 0x7fffffffu, kGuideMulti = 0x80000000u;
 // Unbiased levels whose weight beta^(-e L) / (1 - beta^e) is tabulated.
 constexpr uint32_t kUnbLevels = 32;
@@ -87,6 +88,7 @@ struct PortfolioDevice {
     const StockRec* stocks;
     const double* delta_coalesce;
     const double* chol;  // d x d row-major lower triangle, or nullptr
+    double* chol_room;   // room for chol in the tables' block (d <= kBlobChol; else nullptr)
     uint32_t d;
     double r, rho, s1_rho2, max_loss, tau, stau;
     uint32_t dt_h0inv, dt_beta;
@@ -109,6 +111,27 @@ struct PortfolioDevice {
     uint32_t options_count;
     double prob_norm, total_std;
 };
+
+// Device-side staging (stage.hip): builds the guides and the Exact records from
+// the uploaded options, CDFs and stocks.
+struct StageArgs {
+    const OptionRec* opt1;
+    const double* cdf[3];
+    uint32_t n[3];
+    uint32_t* guide[3];
+    double scale[3];
+    MixRec* mix;
+    ExactRec* ext;
+    const StockRec* stocks;
+    MixStock* ms;
+    ExactStock* es;
+    uint32_t d;
+    double r, tau, stau, prob_norm;
+    int subsample;
+    uint32_t options_count;
+    uint32_t blk[6];  // set by launch_stage
+};
+hipError_t launch_stage(StageArgs A, hipStream_t s);
 
 struct PortfolioParityHost {
     PortfolioDevice pf;

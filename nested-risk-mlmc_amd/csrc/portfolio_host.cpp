@@ -65,7 +65,43 @@ using detail::upload;
 void Engine::free_portfolio() {
     for (void* p : pf_allocs) hipFree(p);
     pf_allocs.clear();
+    if (pf_blob) hipFree(pf_blob);
+    pf_blob = nullptr;
+    pf_blob_cap = 0;
     std::memset(&pf, 0, sizeof(pf));
+}
+
+// Pinned host memory that staging uploads from, kept up to kStageKeep bytes (a
+// larger book's is released with its staging) and given back by
+// cleanup_nestedmc_sampler; stage_ev marks the end of its last upload.
+static constexpr size_t kStageKeep = (size_t)64 << 20;
+
+int Engine::stage_buffer(size_t size) {
+    hipError_t e;
+    if (!stage_ev && (e = hipEventCreateWithFlags(&stage_ev, hipEventDisableTiming)) != hipSuccess)
+        return hip_fail(e, "hipEventCreate staging");
+    if ((e = hipEventSynchronize(stage_ev)) != hipSuccess) return hip_fail(e, "portfolio staging");
+    if (size > h_stage_cap) {
+        if (h_stage) hipHostFree(h_stage);
+        h_stage = nullptr;
+        h_stage_cap = 0;
+        size_t cap = 1 << 20;
+        while (cap < size) cap *= 2;
+        if ((e = hipHostMalloc(&h_stage, cap)) != hipSuccess) return hip_fail(e, "hipHostMalloc staging");
+        h_stage_cap = cap;
+    }
+    return NMLMC_OK;
+}
+
+void Engine::free_stage() {
+    if (stage_ev) {
+        hipEventSynchronize(stage_ev);
+        hipEventDestroy(stage_ev);
+    }
+    if (h_stage) hipHostFree(h_stage);
+    stage_ev = nullptr;
+    h_stage = nullptr;
+    h_stage_cap = 0;
 }
 
 // portfolio_update_data (portfolio_sampler.cpp:631-678).
@@ -80,23 +116,52 @@ int Engine::stage_portfolio(const portfolio_data* data) {
     const uint32_t ps = (data->phi_type == 0 || data->phi_type == 1) ? 1u : data->_phi_size;
     if (ps == 0 || ps > (uint32_t)kMaxPhi) return set_error(NMLMC_ERR_ARG, "phi size must be 1..4");
     if (ensure_device()) return nmlmc_last_error();
-    free_portfolio();
+    // One block of device memory holds every table.  The uploaded part (options,
+    // CDFs, stocks, coalesced deltas) comes first and is filled in pinned host
+    // memory; the rest is built by k_stage from it, and room for a Cholesky factor
+    // of up to kBlobChol stocks follows.
+    static_assert(sizeof(option_params) == sizeof(OptionRec), "option record layout");
+    static_assert(sizeof(stock_params) == sizeof(StockRec), "stock record layout");
+    size_t size = 0;
+    auto take = [&size](size_t bytes) {
+        const size_t off = size;
+        size = (size + bytes + 255) & ~(size_t)255;
+        return off;
+    };
+    size_t n[3], o_opt[3], o_cdf[3], o_guide[3];
+    for (int m = 0; m < 3; m++) {
+        n[m] = data->options[m].size;
+        if (n[m] && !data->options[m].data) return set_error(NMLMC_ERR_ARG, "options[%d] is NULL", m);
+        if (n[m] > kGuideLo / 4) return set_error(NMLMC_ERR_ARG, "options[%d]: too many options", m);
+        o_opt[m] = take(sizeof(OptionRec) * n[m]);
+        o_cdf[m] = take(sizeof(double) * n[m]);
+    }
+    const size_t o_stocks = take(sizeof(StockRec) * d), o_delta = take(sizeof(double) * d);
+    const size_t up = size;
+    for (int m = 0; m < 3; m++) o_guide[m] = take(n[m] ? sizeof(uint32_t) * (4 * n[m] + 1) : 0);
+    const size_t o_mix = take(sizeof(MixRec) * n[1]), o_ext = take(sizeof(ExactRec) * n[1]),
+                 o_ms = take(sizeof(MixStock) * d), o_es = take(sizeof(ExactStock) * d);
+    const size_t o_chol = take(d <= kBlobChol ? sizeof(double) * d * d : 0);
+    int rc = stage_buffer(up);
+    if (rc) return rc;
+    char* const host = (char*)h_stage;
     PortfolioDevice P;
     std::memset(&P, 0, sizeof(P));
     const stock_params* stocks = (const stock_params*)data->stocks.data;
-    std::vector<double> delta(d, 0.);
+    double* delta = (double*)(host + o_delta);
+    for (uint32_t i = 0; i < d; i++) delta[i] = 0.;
     P.prob_norm = 0;
     P.total_std = 0;
     P.options_count = 0;
+    double w_est0 = 0.;
+    bool w_est_same = true;
     for (int m = 0; m < 3; m++) {
         const option_params* ops = (const option_params*)data->options[m].data;
-        const size_t n = data->options[m].size;
-        if (n && !ops) return set_error(NMLMC_ERR_ARG, "options[%d] is NULL", m);
-        std::vector<double> cdf(n);
+        double* cdf = (double*)(host + o_cdf[m]);
         double c = 0;
         double prev = 1.7976931348623157e308;
         P.compute_prob[m] = 0;
-        for (size_t j = 0; j < n; j++) {
+        for (size_t j = 0; j < n[m]; j++) {
             const option_params& o = ops[j];
             if (!(o.prob > 0 && prev >= o.prob))
                 return set_error(NMLMC_ERR_ARG, "options[%d][%zu]: probabilities must be positive and "
@@ -114,49 +179,20 @@ int Engine::stage_portfolio(const portfolio_data* data) {
             P.prob_norm += o.prob;
             P.total_std += o.prob * o.W_est;
             P.compute_prob[m] += o.prob;
+            if (P.options_count == 0 && j == 0) w_est0 = o.W_est;
+            w_est_same = w_est_same && o.W_est == w_est0;
         }
-        static_assert(sizeof(option_params) == sizeof(OptionRec), "option record layout");
-        int rc = upload(*this, (const OptionRec*)ops, n, &P.options[m]);
-        if (rc) return rc;
-        if ((rc = upload(*this, cdf.data(), n, &P.cdfs[m]))) return rc;
-        // Guide of the option search: nb = 4n buckets; bucket b holds the u with
-        // (uint32)(u * scale) == b, i.e. [edge(b), edge(b + 1)) with edge(b) the
-        // smallest double whose product with scale (one IEEE multiply, as on the
-        // device) reaches b; its entry is the answer at both edges.
-        if (n) {
-            const uint64_t nb = 4 * (uint64_t)n;
-            const double scale = (double)nb / c;
-            auto edge = [scale](uint64_t b) {
-                if (b == 0) return 0.;
-                double x = (double)b / scale;
-                while (x > 0 && std::nextafter(x, 0.) * scale >= (double)b) x = std::nextafter(x, 0.);
-                while (x * scale < (double)b) x = std::nextafter(x, 1e308);
-                return x;
-            };
-            std::vector<uint32_t> at(nb + 1);
-            size_t i = 0;
-            for (uint64_t b = 0; b < nb; b++) {
-                const double x = edge(b);
-                while (i + 1 < n && cdf[i + 1] <= x) i++;
-                at[b] = (uint32_t)i;
-            }
-            at[nb] = (uint32_t)(n - 1);  // the last bucket is open above
-            if (n > kGuideLo) return set_error(NMLMC_ERR_ARG, "options[%d]: too many options", m);
-            std::vector<uint32_t> guide(nb + 1);
-            for (uint64_t b = 0; b < nb; b++) guide[b] = at[b] | (at[b + 1] != at[b] ? kGuideMulti : 0u);
-            guide[nb] = at[nb];
-            if ((rc = upload(*this, guide.data(), nb + 1, &P.guides[m]))) return rc;
-            P.guide_scale[m] = scale;
-            P.guide_nb[m] = (uint32_t)nb;
+        if (n[m]) {
+            std::memcpy(host + o_opt[m], ops, sizeof(OptionRec) * n[m]);
+            P.guide_nb[m] = (uint32_t)(4 * n[m]);
+            P.guide_scale[m] = (double)(4 * n[m]) / c;
         }
-        P.nopt[m] = (uint32_t)n;
-        P.options_count += (uint32_t)n;
+        P.nopt[m] = (uint32_t)n[m];
+        P.options_count += (uint32_t)n[m];
     }
     if (P.options_count == 0) return set_error(NMLMC_ERR_ARG, "portfolio has no options");
-    static_assert(sizeof(stock_params) == sizeof(StockRec), "stock record layout");
-    int rc = upload(*this, (const StockRec*)stocks, d, &P.stocks);
-    if (rc) return rc;
-    if ((rc = upload(*this, delta.data(), d, &P.delta_coalesce))) return rc;
+    P.w_est_const = w_est_same ? w_est0 : -1.;
+    std::memcpy(host + o_stocks, stocks, sizeof(StockRec) * d);
     P.chol = nullptr;
     P.d = d;
     P.r = data->r;
@@ -184,62 +220,46 @@ int Engine::stage_portfolio(const portfolio_data* data) {
     P.coupled = (level_coupled && data->options[2].size) ? 1u : 0u;
     if (P.coupled && data->subsample != 1)
         return set_error(NMLMC_ERR_ARG, "level-coupled paths need sub-sampling mode 1");
-    // Records of the Exact options and of the stocks for the mixed (FP32) and the
-    // FP64 inner terms, in one upload.
-    {
-        const option_params* ex = (const option_params*)data->options[1].data;
-        const size_t n1 = data->options[1].size;
-        auto at = [](size_t off) { return (off + 63) & ~(size_t)63; };
-        const size_t o_ext = at(sizeof(MixRec) * n1), o_ms = at(o_ext + sizeof(ExactRec) * n1),
-                     o_es = at(o_ms + sizeof(MixStock) * d), size = o_es + sizeof(ExactStock) * d;
-        std::vector<char> tab(size, 0);
-        MixRec* mix = (MixRec*)tab.data();
-        ExactRec* ext = (ExactRec*)(tab.data() + o_ext);
-        MixStock* ms = (MixStock*)(tab.data() + o_ms);
-        ExactStock* es = (ExactStock*)(tab.data() + o_es);
-        for (size_t j = 0; j < n1; j++) {
-            const option_params& o = ex[j];
-            const double w = o.w * std::exp(-data->r * o.maturity);
-            const double Tt = o.maturity - data->tau, sTt = std::sqrt(Tt);
-            const uint32_t stype = (o.stock_ind << 8) | (uint32_t)(o.type + 2);
-            mix[j] = MixRec{(float)o.strike, (float)sTt, (float)(w * P.prob_norm / o.prob), stype};
-            const double discp = data->subsample == 1    ? w / (o.prob / P.prob_norm)
-                                 : data->subsample == -1 ? w * P.options_count
-                                                         : w;
-            ext[j] = ExactRec{o.strike, Tt, sTt, discp, stype, 0};
-        }
-        for (uint32_t i = 0; i < d; i++) {
-            const stock_params& st = stocks[i];
-            const double dcoef = data->r - 0.5 * st.sigma * st.sigma;
-            MixStock& q = ms[i];
-            q.sig = (float)st.sigma;
-            q.dcoef = (float)dcoef;
-            q.sigtau = (float)(st.sigma * std::sqrt(data->tau));
-            q.S0e = (float)(st.S0 * std::exp(dcoef * data->tau));
-            q.S0 = (float)st.S0;
-            q.invS0 = (float)(1. / st.S0);
-            es[i] = ExactStock{st.sigma, dcoef, dcoef * data->tau, P.stau, st.S0, 1. / st.S0};
-        }
-        const char* dev;
-        if ((rc = upload(*this, (const char*)tab.data(), size, &dev))) return rc;
-        P.mix = (const MixRec*)dev;
-        P.exact = (const ExactRec*)(dev + o_ext);
-        P.mix_stocks = (const MixStock*)(dev + o_ms);
-        P.exact_stocks = (const ExactStock*)(dev + o_es);
+    // The book is valid: its tables replace the staged ones.  The block is used again
+    // when it fits (work on the tables is ordered on the engine's stream).
+    for (void* p : pf_allocs) hipFree(p);
+    pf_allocs.clear();
+    hipError_t e;
+    if (size > pf_blob_cap || pf_blob_cap > 4 * size + ((size_t)1 << 20)) {
+        free_portfolio();
+        problem = -1;  // nothing is staged if the allocation fails
+        if ((e = hipMalloc(&pf_blob, size)) != hipSuccess) return hip_fail(e, "hipMalloc portfolio tables");
+        pf_blob_cap = size;
     }
-    P.w_est_const = -1.;
-    {
-        bool first = true, same = true;
-        double w0 = 0.;
-        for (int m = 0; m < 3; m++) {
-            const option_params* ops = (const option_params*)data->options[m].data;
-            for (size_t j = 0; j < data->options[m].size; j++) {
-                if (first) w0 = ops[j].W_est, first = false;
-                else same = same && ops[j].W_est == w0;
-            }
-        }
-        if (!first && same) P.w_est_const = w0;
+    char* const dev = (char*)pf_blob;
+    if ((e = hipMemcpyAsync(dev, host, up, hipMemcpyHostToDevice, stream)) != hipSuccess)
+        return hip_fail(e, "hipMemcpy portfolio tables");
+    StageArgs S{};
+    for (int m = 0; m < 3; m++) {
+        P.options[m] = (const OptionRec*)(dev + o_opt[m]);
+        P.cdfs[m] = S.cdf[m] = (const double*)(dev + o_cdf[m]);
+        P.guides[m] = S.guide[m] = (uint32_t*)(dev + o_guide[m]);
+        S.n[m] = P.nopt[m];
+        S.scale[m] = P.guide_scale[m];
     }
+    P.stocks = S.stocks = (const StockRec*)(dev + o_stocks);
+    P.delta_coalesce = (const double*)(dev + o_delta);
+    P.mix = S.mix = (MixRec*)(dev + o_mix);
+    P.exact = S.ext = (ExactRec*)(dev + o_ext);
+    P.mix_stocks = S.ms = (MixStock*)(dev + o_ms);
+    P.exact_stocks = S.es = (ExactStock*)(dev + o_es);
+    P.chol_room = d <= kBlobChol ? (double*)(dev + o_chol) : nullptr;
+    S.opt1 = P.options[1];
+    S.d = d;
+    S.r = P.r;
+    S.tau = P.tau;
+    S.stau = P.stau;
+    S.prob_norm = P.prob_norm;
+    S.subsample = P.subsample;
+    S.options_count = P.options_count;
+    if ((e = launch_stage(S, stream)) != hipSuccess) return hip_fail(e, "launch k_stage");
+    if ((e = hipEventRecord(stage_ev, stream)) != hipSuccess) return hip_fail(e, "hipEventRecord staging");
+    if (h_stage_cap > kStageKeep) free_stage();
     // Work of one init_inner_sampler call without sub-sampling: the BS options.
     pf_bs_work = 0.;
     if (data->subsample == 0) {
@@ -502,6 +522,12 @@ int nmlmc_portfolio_set_correlation(const double* chol, uint32_t d) {
         return set_error(NMLMC_OK, "");
     }
     if (d != g_engine.pf.d) return set_error(NMLMC_ERR_ARG, "correlation factor must be %u x %u", g_engine.pf.d, g_engine.pf.d);
+    if (g_engine.pf.chol_room) {
+        const hipError_t e = hipMemcpy(g_engine.pf.chol_room, chol, sizeof(double) * d * d, hipMemcpyHostToDevice);
+        if (e != hipSuccess) return nmlmc::hip_fail(e, "hipMemcpy correlation factor");
+        g_engine.pf.chol = g_engine.pf.chol_room;
+        return set_error(NMLMC_OK, "");
+    }
     const double* p = nullptr;
     int rc = nmlmc::detail::upload(g_engine, chol, (size_t)d * d, &p);
     if (rc) return rc;
