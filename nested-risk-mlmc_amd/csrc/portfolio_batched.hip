@@ -191,7 +191,8 @@ struct PortfolioPolicyT {
                 pick_option(pf, st, st, method, idx);
                 const OptionRec o = pf.options[2][idx];
                 prob = option_prob(pf, o);
-                unbiased_begin(pf, o, R, st, st, work, p);
+                const uint32_t L = unbiased_level(pf, st.randu());
+                unbiased_begin(pf, o, R, L, st.randn(), work, p);
                 // simulate_dt_d's step sizes
                 const double t = o.maturity - pf.tau;
                 sigma = pf.stocks[o.stock_ind].sigma;
@@ -372,7 +373,7 @@ struct PortfolioPolicyT {
                         continue;
                     }
                     if (method == 2) {
-                        const uint32_t L = unbiased_level(pf, st);
+                        const uint32_t L = unbiased_level(pf, st.randu());
                         const uint64_t bit = 1ull << j;
                         if (L == 0) lv0 |= bit;
                         else if (L == 1) lv1 |= bit;

@@ -144,8 +144,9 @@ __device__ __forceinline__ double inner_exact_d(const ExactRec& q, const ExactSt
 // simulate_stock_dt (gbm_approx.hpp:18-57) for 3 fine (+ 3 coarse) paths.
 // AVG (the Asian extension): A[i] becomes the average of path i's values after
 // each of its steps (fine: N steps, coarse: N / coarse_step), in step order.
-template <bool AVG>
-__device__ __forceinline__ void simulate_dt_d(DStream& rn, double* S, double* A, uint64_t N, double mu,
+// rn.randn() gives the paths' normals in order.
+template <bool AVG, class RN>
+__device__ __forceinline__ void simulate_dt_d(RN& rn, double* S, double* A, uint64_t N, double mu,
                                               double sigma, double t, bool with_coarse, bool milstein,
                                               uint32_t coarse_step) {
     const double dt = t / (double)N;
@@ -226,12 +227,12 @@ __device__ __forceinline__ uint64_t upow(uint64_t x, uint64_t n) {
 // The randomised level of an Unbiased inner sample (sample_inner_unbiased,
 // 521-537): L = floor(ln u / (ln beta * e)) from one sync uniform, so that
 // P(L >= l) = beta^(e l).
-__device__ __forceinline__ uint32_t unbiased_level(const PortfolioDevice& pf, DStream& sync) {
-    return (uint32_t)floor(log(sync.randu()) / pf.unb_lnbe);
+__device__ __forceinline__ uint32_t unbiased_level(const PortfolioDevice& pf, double u) {
+    return (uint32_t)floor(log(u) / pf.unb_lnbe);
 }
 
-// One Unbiased inner sample in three parts: unbiased_begin draws its level and
-// initial increment and sets the paths' values at tau (3 fine paths: S0 and its
+// One Unbiased inner sample of level L in three parts: unbiased_begin takes its
+// initial increment's normal and sets the paths' values at tau (3 fine paths: S0 and its
 // antithetic twin to tau, and the outer sample's level; the same 3 coarse);
 // the paths then run N fine (N / beta coarse) Milstein steps, in one lane
 // (simulate_dt_d) or split over a wave; unbiased_end prices the options on them.
@@ -243,12 +244,12 @@ struct UnbiasedPath {
 
 // sample_inner_approx (539-604) up to its call of simulate_stock_dt.
 template <class RT>
-__device__ __forceinline__ void unbiased_begin(const PortfolioDevice& pf, const OptionRec& o, RT R_tau, DStream& sync,
-                                               DStream& inner, double& work, UnbiasedPath& p) {
-    p.L = unbiased_level(pf, sync);
+__device__ __forceinline__ void unbiased_begin(const PortfolioDevice& pf, const OptionRec& o, RT R_tau, uint32_t L,
+                                               double z, double& work, UnbiasedPath& p) {
+    p.L = L;
     const uint32_t si = o.stock_ind;
     const StockRec st = pf.stocks[si];
-    const double dW_0_tau = pf.stau * inner.randn();
+    const double dW_0_tau = pf.stau * z;
     const double S0_t_1 = simulate_stock_d(st.S0, pf.r, st.sigma, pf.tau, dW_0_tau);
     const double S0_t_2 = simulate_stock_d(st.S0, pf.r, st.sigma, pf.tau, -dW_0_tau);
     const uint64_t N_l = upow(pf.dt_beta, p.L);
@@ -289,13 +290,13 @@ __device__ __forceinline__ double unbiased_end(const PortfolioDevice& pf, const 
     return ret * L_prob_1;
 }
 
-// sample_inner_unbiased (521-537) + sample_inner_approx (539-604), the paths in
-// this lane.
-template <class RT>
-__device__ __forceinline__ double inner_unbiased_d(const PortfolioDevice& pf, const OptionRec& o, RT R_tau,
-                                                   DStream& sync, DStream& inner, double& work) {
+// sample_inner_unbiased (521-537) + sample_inner_approx (539-604) at level L, the
+// paths in this lane.
+template <class RT, class RN>
+__device__ __forceinline__ double inner_unbiased_at(const PortfolioDevice& pf, const OptionRec& o, RT R_tau,
+                                                    uint32_t L, RN& inner, double& work) {
     UnbiasedPath p;
-    unbiased_begin(pf, o, R_tau, sync, inner, work, p);
+    unbiased_begin(pf, o, R_tau, L, inner.randn(), work, p);
     const StockRec st = pf.stocks[o.stock_ind];
     const double T_tau = o.maturity - pf.tau;
     const bool asian = is_asian(o.type);
@@ -307,6 +308,12 @@ __device__ __forceinline__ double inner_unbiased_d(const PortfolioDevice& pf, co
         else simulate_dt_d<false>(inner, p.S, p.A, p.N, pf.r, st.sigma, T_tau, false, pf.use_milstein, 2);
     }
     return unbiased_end(pf, o, R_tau, p);
+}
+template <class RT>
+__device__ __forceinline__ double inner_unbiased_d(const PortfolioDevice& pf, const OptionRec& o, RT R_tau,
+                                                   DStream& sync, DStream& inner, double& work) {
+    const uint32_t L = unbiased_level(pf, sync.randu());
+    return inner_unbiased_at(pf, o, R_tau, L, inner, work);
 }
 
 // Steps of the level-coupled paths at level l: dt_h0inv 2^floor(l / 2).

@@ -11,8 +11,11 @@
 //     (Exact: option uniform + one Box-Muller pair) inner words; lanes take
 //     chunks of 64 samples and find their inner word offsets by a ballot
 //     prefix count, so every draw matches the sequential reference;
-//   - other configurations (no sub-sampling, Unbiased options, a cached inner
-//     normal) run the reference loop on thread 0.
+//   - an inner loop with Unbiased options finds its samples' positions in the two
+//     streams by windows of 64 sync words and evaluates them on all lanes
+//     (general_inner);
+//   - other configurations (no sub-sampling, or a cached inner normal in a book
+//     without Unbiased options) run the reference loop on thread 0.
 // A virtual thread may take a block of W <= 8 waves (W > 1 only for books whose
 // options are all Exact, chosen when few virtual threads have outer samples):
 // the outer draw's stocks and the inner loop's samples are then spread over
@@ -61,6 +64,292 @@ __device__ __forceinline__ double phi_value(int phi_type, double u, double coeff
 // no BS or Unbiased code; books without Unbiased options.  Leaving code out
 // keeps a kernel to a fraction of the general one's registers.
 enum { PAR_GENERAL = 0, PAR_EXACT = 1, PAR_NO_UNBIASED = 2 };
+
+// The inner loop of a sub-sampled book with Unbiased options, on one wave.  A
+// sample's draws depend on its own draws: its method is one sync word and, when
+// that is Unbiased, its level the next; its normals are 2 (Exact) or 1 + N
+// (Unbiased, N steps at its level) of the inner stream after one word for the
+// option, drawn in pairs whose second normal waits for the next sample that needs
+// one.  But the words that set these positions are few, so the wave takes the
+// samples by windows of 64 sync words:
+//   - every lane evaluates its word both as a method and as a level; the samples'
+//     first words follow from the mask of Unbiased methods (a word after the
+//     method of an Unbiased sample is its level);
+//   - lanes that hold a sample get its inner words by a prefix sum (whether a
+//     normal waits is the parity of the odd draws before it), and its waiting
+//     normal from the words of the last pair drawn before it;
+//   - Black-Scholes and Exact samples are then evaluated side by side;
+//   - the normals of the Unbiased samples with at most kFlat pairs (levels 0
+//     and 1 by default) are computed as one list spread over all lanes, into LDS,
+//     and each sample's paths run in its lane;
+//   - the longer ones follow one at a time: all lanes compute the path factors of
+//     kBatch steps, and six lanes run the six paths on them.
+// Draws, and every operation within a sample, are those of the sequence on one
+// lane; only the order of the samples' sums differs.
+//
+// On one lane (63 idle) a sample took some 1500 dependent instructions: the mix of
+// the reference's own main (1000 options, levels 0..3, 8192 outer samples at level 0)
+// 43 ms a sweep, 7.1 ms this way.
+struct GeneralScratch {
+    static constexpr uint32_t kFlat = 20;    // pairs of a sample of the flat list
+    static constexpr uint32_t kPairs = 384;  // the list's buffer
+    static constexpr uint32_t kBatch = 126;  // steps of a long path at a time (rounded down to whole coarse steps)
+    double z[2 * kPairs];                    // normals; long paths: dW
+    double g[kBatch], gc[kBatch];            // long paths: fine and coarse step factors
+    uint8_t owner[kPairs];
+};
+
+struct LdsNormals {
+    const double* z;
+    double first;
+    bool has_first;
+    __device__ __forceinline__ double randn() {
+        if (has_first) {
+            has_first = false;
+            return first;
+        }
+        return *z++;
+    }
+};
+
+__device__ __forceinline__ void lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The long paths of lane ow's sample (level p.L, p.N steps; normals from inner
+// word Pn, the first of them the waiting one when sb), over the wave; the owner's p
+// gets the values at T and, for Asians, the averages.
+__device__ __forceinline__ void long_paths(const PortfolioDevice& pf, uint64_t seed, uint64_t k1, uint32_t ow,
+                                           uint64_t Pn, uint32_t sb, double sigma, double T, GeneralScratch& sc,
+                                           UnbiasedPath& p) {
+    const uint32_t lane = threadIdx.x & 63;
+    Pn = bcast_u64(Pn, ow);
+    sb = bcast_u32(sb, ow);
+    const uint64_t N = bcast_u64(p.N, ow);
+    const bool coarse = bcast_u32(p.L, ow) != 0;
+    const uint32_t beta = coarse ? pf.dt_beta : 1;
+    const double sg = bcast_f64(sigma, ow), t = bcast_f64(T, ow);
+    const double mu = pf.r, dt = t / (double)N, sqrt_dt = sqrt(dt), dt_c = t / (double)(N / beta);
+    const bool milstein = pf.use_milstein;
+    double S = 0., A = 0.;  // lane i < 6: path i
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        const double v = bcast_f64(p.S[i], ow);
+        if (lane == (uint32_t)i) S = v;
+    }
+    const uint32_t per = GeneralScratch::kBatch - GeneralScratch::kBatch % beta;
+    for (uint64_t s0 = 0; s0 < N; s0 += per) {
+        const uint32_t n = (uint32_t)(N - s0 < per ? N - s0 : per);
+        // Step s uses normal s + 1 of the sample, number s + 1 - sb of its pairs.
+        const uint64_t first = (s0 + 1 - sb) >> 1, last = (s0 + n - sb) >> 1;
+        const uint64_t b = first + lane;
+        if (b <= last) {  // at most 64 pairs
+            double x, y;
+            stream_bm_f64(seed, k1, Pn + 2 * b, x, y);
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const uint64_t num = 2 * b + e + sb;  // the sample's normal number
+                if (num >= s0 + 1 && num <= s0 + n) {
+                    const uint32_t k = (uint32_t)(num - 1 - s0);
+                    const double dW = sqrt_dt * (e ? y : x);
+                    const double m = milstein ? (0.5 * (sg * sg) * (dW * dW - dt)) : 0.;
+                    sc.z[k] = dW;
+                    sc.g[k] = mu * dt + sg * dW + m;
+                }
+            }
+        }
+        lds_fence();
+        if (coarse) {
+            for (uint32_t c = lane; c < n / beta; c += 64) {
+                double dW_c = 0.;
+                for (uint32_t i = 0; i < beta; i++) dW_c += sc.z[c * beta + i];
+                const double m = milstein ? (0.5 * (sg * sg) * (dW_c * dW_c - dt_c)) : 0.;
+                sc.gc[c] = mu * dt_c + sg * dW_c + m;
+            }
+            lds_fence();
+        }
+        const double* f = lane < 3 ? sc.g : sc.gc;
+        const uint32_t len = lane < 3 ? n : (coarse ? n / beta : 0);
+        if (lane < 6)
+            for (uint32_t k = 0; k < len; k++) {
+                S += S * f[k];
+                A += S;
+            }
+        lds_fence();
+    }
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        const double v = bcast_f64(S, i), a = bcast_f64(A, i);
+        if (lane == ow) {
+            p.S[i] = v;
+            if (i < 3 || coarse) p.A[i] = a / (double)(i < 3 ? N : N / beta);
+        }
+    }
+}
+
+__device__ __forceinline__ InnerSums general_inner(const PortfolioParityArgs& A, const double* R, uint64_t k1,
+                                                   StreamState& ss, StreamState& si, uint64_t count,
+                                                   GeneralScratch& sc) {
+    const PortfolioDevice& pf = A.pf;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    double s1 = 0., s2 = 0., work = 0.;
+    uint64_t nu = 0, nn = 0;
+    // The waiting normal: known (si.saved), or the second of the pair at word wait_pos.
+    uint32_t wait = si.is_saved;
+    bool wait_known = true;
+    uint64_t wait_pos = 0;
+    auto add = [&](double v) {
+        s1 += v;
+        s2 += v * v;
+    };
+    for (uint64_t done = 0; done < count;) {
+        const double uw = u01_f64(stream_word(A.seed, k1, ss.P + lane));
+        const uint32_t method = pick_method(pf, uw * pf.prob_norm);
+        const uint32_t level = unbiased_level(pf, uw);
+        // Samples whose words all lie in the window, in order, at most those left.
+        const uint64_t two = __ballot(method == 2), left = count - done;
+        uint64_t starts = 0;
+        uint32_t pos = 0, n = 0;
+        while (pos < 63 && n < left) {
+            const uint64_t rest = two >> pos;
+            const uint32_t to2 = rest ? pos + (uint32_t)__builtin_ctzll(rest) : 64u;
+            uint32_t run = (to2 < 63 ? to2 : 63) - pos;  // one-word samples before it
+            if (run > left - n) run = (uint32_t)(left - n);
+            if (run) starts |= (~0ull >> (64 - run)) << pos;
+            pos += run;
+            n += run;
+            if (n < left && pos == to2 && pos < 63) {
+                starts |= 1ull << pos;
+                pos += 2;
+                n++;
+            }
+        }
+        ss.P += pos;
+        done += n;
+        const bool mine = (starts >> lane) & 1;
+        const uint32_t L = (uint32_t)__shfl((int)level, (int)((lane + 1) & 63), 64);
+        const bool bs = mine && method == 0, exact = mine && method == 1, unb = mine && method == 2;
+        const uint64_t N = unb ? (uint64_t)pf.dt_h0inv * upow(pf.dt_beta, L) : 0;
+        // Whether a normal waits before the sample; its inner words.
+        const uint64_t odd = __ballot(unb && ((1 + N) & 1));
+        const uint32_t sb = wait ^ ((uint32_t)__popcll(odd & below) & 1u);
+        const uint64_t pairs = exact ? 1 : unb ? (1 + N - sb + 1) / 2 : 0;
+        uint64_t end = mine ? 1 + 2 * pairs : 0;  // inclusive prefix sum of the words
+#pragma unroll
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint64_t v = __shfl_up((unsigned long long)end, o, 64);
+            if (lane >= o) end += v;
+        }
+        const uint64_t total = bcast_u64(end, 63);
+        end += si.P;
+        const uint64_t Pn = end - 2 * pairs;  // the sample's first normal's word
+        const uint64_t drew = __ballot(pairs != 0);
+        const uint64_t before = drew & below;
+        const uint32_t prev = before ? 63u - (uint32_t)__clzll((long long)before) : 0u;
+        const uint64_t prev_end = __shfl((unsigned long long)end, (int)prev, 64);
+        double w = si.saved;
+        if ((exact || unb) && sb && (before || !wait_known)) {
+            double x;
+            stream_bm_f64(A.seed, k1, before ? prev_end - 2 : wait_pos, x, w);
+        }
+        if (mine) {
+            nu += unb ? 3 : 2;
+            nn += exact ? 2 : unb ? 1 + N : 0;
+        }
+        uint32_t idx = 0;
+        if (mine) idx = pick_in_method(pf, method, u01_f64(stream_word(A.seed, k1, Pn - 1)));
+        if (exact) {
+            double x, y;
+            stream_bm_f64(A.seed, k1, Pn, x, y);
+            add(exact_term(pf, idx, R, sb ? w : x, sb ? x : y, work));
+        }
+        if (bs) {
+            const OptionRec o = pf.options[0][idx];
+            add(inner_bs_d(pf, o, R, work) / option_prob(pf, o));
+        }
+        // Unbiased samples of few pairs: their normals as one list.
+        const bool flat = unb && pairs <= GeneralScratch::kFlat;
+        uint32_t off = flat ? (uint32_t)pairs : 0;  // inclusive prefix sum of the pairs
+#pragma unroll
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)off, o, 64);
+            if (lane >= o) off += v;
+        }
+        if (flat) off -= (uint32_t)pairs;
+        for (uint64_t rem = __ballot(flat); rem;) {
+            const uint32_t base = bcast_u32(off, (uint32_t)__builtin_ctzll(rem));
+            const bool sel = ((rem >> lane) & 1) && off + (uint32_t)pairs - base <= GeneralScratch::kPairs;
+            const uint64_t smask = __ballot(sel);  // the first of rem always fits
+            const uint32_t lastl = 63u - (uint32_t)__clzll((long long)smask);
+            const uint32_t cnt = bcast_u32(off + (uint32_t)pairs, lastl) - base;
+            rem &= ~smask;
+            if (sel)
+                for (uint32_t k = 0; k < (uint32_t)pairs; k++) sc.owner[off - base + k] = (uint8_t)lane;
+            lds_fence();
+            for (uint32_t c0 = 0; c0 < cnt; c0 += 64) {
+                const uint32_t c = c0 + lane;
+                const int o = c < cnt ? (int)sc.owner[c] : (int)lane;
+                const uint64_t oP = __shfl((unsigned long long)Pn, o, 64);
+                const uint32_t oo = (uint32_t)__shfl((int)off, o, 64) - base;
+                if (c < cnt) stream_bm_f64(A.seed, k1, oP + 2 * (uint64_t)(c - oo), sc.z[2 * c], sc.z[2 * c + 1]);
+            }
+            lds_fence();
+            if (sel) {
+                LdsNormals ln{sc.z + 2 * (off - base), w, sb != 0};
+                const OptionRec o = pf.options[2][idx];
+                add(inner_unbiased_at(pf, o, R, L, ln, work) / option_prob(pf, o));
+            }
+            lds_fence();
+        }
+        // Longer ones, one at a time.
+        for (uint64_t rem = __ballot(unb && !flat); rem; rem &= rem - 1) {
+            const uint32_t ow = (uint32_t)__builtin_ctzll(rem);
+            const bool me = lane == ow;
+            UnbiasedPath p;
+            p.L = 0;
+            p.N = 1;
+            double sigma = 0., T = 1.;
+            OptionRec o{};
+            if (pf.dt_beta > GeneralScratch::kBatch) {  // coarse steps longer than a batch: in the lane
+                if (me) {
+                    DStream in;
+                    in.init(A.seed, k1, 0, Pn, w, sb);
+                    o = pf.options[2][idx];
+                    add(inner_unbiased_at(pf, o, R, L, in, work) / option_prob(pf, o));
+                }
+                continue;
+            }
+            if (me) {
+                o = pf.options[2][idx];
+                double z = w;
+                if (!sb) {
+                    double y;
+                    stream_bm_f64(A.seed, k1, Pn, z, y);
+                }
+                unbiased_begin(pf, o, R, L, z, work, p);
+                sigma = pf.stocks[o.stock_ind].sigma;
+                T = o.maturity - pf.tau;
+            }
+            long_paths(pf, A.seed, k1, ow, Pn, sb, sigma, T, sc, p);
+            if (me) add(unbiased_end(pf, o, R, p) / option_prob(pf, o));
+        }
+        si.P += total;
+        wait ^= (uint32_t)__popcll(odd) & 1u;
+        if (drew) {
+            wait_known = false;
+            wait_pos = bcast_u64(end, 63u - (uint32_t)__clzll((long long)drew)) - 2;
+        }
+    }
+    if (wait && !wait_known) {
+        double x, y;
+        stream_bm_f64(A.seed, k1, wait_pos, x, y);
+        si.saved = y;
+    }
+    si.is_saved = wait;
+    return InnerSums{wave_sum(s1), wave_sum(s2), wave_sum(work), wave_sum_u64(nu), wave_sum_u64(nn)};
+}
 
 // inner_sampler::sample_inner (nested_sampler.hpp:131-161) over `count` samples
 // from the thread's streams (ss: sync, si: inner), block-uniform result.  red:
@@ -141,6 +430,11 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
         ss.P += count;
         si.P += base;
         return r;
+    }
+    if constexpr (KIND == PAR_GENERAL) {
+        static_assert(W == 1, "one wave a virtual thread");
+        __shared__ GeneralScratch sc;
+        if (pf.subsample != 0) return general_inner(A, R, k1, ss, si, count, sc);
     }
     // Reference loop on thread 0.
     if (tid == 0) {
