@@ -24,24 +24,23 @@ struct StockRec {
 };
 
 // data_ex (portfolio_sampler.cpp:94-132) with device pointers.
-// One Exact option for the FP32 inner loop of the mixed form (16 bytes).
+// One Exact option for the FP32 inner loop of the mixed form (16 bytes).  Stock
+// levels and strikes are in units of the stock's S0, so that a stock needs four
+// constants (one load) and no division.
 struct MixRec {
-    float K;         // strike
+    float K;         // strike / S0
     float sTt;       // sqrt(T - tau)
-    float discp;     // w e^{-rT} / p, p = prob / prob_norm
+    float hdiscp;    // w e^{-rT} / (2 p), p = prob / prob_norm, times S0 unless the option is a digital
     uint32_t stype;  // stock index << 8 | (type + 2)
 };
 static_assert(sizeof(MixRec) == 16, "mixed option record must stay 16 bytes");
 
-// Per-stock constants of the mixed form's inner loop (32 bytes).
-struct MixStock {
-    float sig;     // sigma
-    float dcoef;   // r - sigma^2 / 2
-    float sigtau;  // sigma sqrt(tau)
-    float S0e;     // S0 e^{(r - sigma^2 / 2) tau}
-    float S0;      // S0
-    float invS0;   // 1 / S0 (the control variate's S / S0 as a product)
-    float pad[2];
+// Per-stock constants of the mixed form's inner loop (16 bytes); exponents to base 2.
+struct alignas(16) MixStock {
+    float sig;     // sigma log2 e
+    float dcoef;   // (r - sigma^2 / 2) log2 e
+    float sigtau;  // sigma sqrt(tau) log2 e
+    float S0e;     // e^{(r - sigma^2 / 2) tau}
 };
 
 // One Exact option for the FP64 inner term (40 of an OptionRec's 64 bytes).

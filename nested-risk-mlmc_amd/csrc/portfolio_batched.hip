@@ -28,7 +28,7 @@ struct PortfolioPolicyT {
         double* R_tau;  // [M x d] (MULTI: [M x dmax]): stock i of outer sample m at R_tau[m * stride + i]
         double bs_work; // work of one init_inner_sampler call (sub-sampling off)
         PortfolioBatchTables bt;
-        float* R32;     // mixed Exact-only form: FP32 copies of R_tau, same layout (else NULL)
+        float* R32;     // mixed Exact-only form: R_tau over S0 in FP32, same layout (else NULL)
     };
     static constexpr uint64_t spu = 1;
     static constexpr bool kMulti = MULTI;
@@ -126,7 +126,7 @@ struct PortfolioPolicyT {
             if (pf.d == 1) {
                 const StockRec st = pf.stocks[0];
                 Rw[0] = simulate_stock_d(st.S0, st.mu, st.sigma, pf.tau, dW_sys);
-                if (Rw32) Rw32[0] = (float)Rw[0];
+                if (Rw32) Rw32[0] = (float)(Rw[0] / st.S0);
             } else {
                 for (uint32_t i = 0; i < pf.d; i++) {
                     const double dW_ind = pf.stau * os.randn();
@@ -134,7 +134,7 @@ struct PortfolioPolicyT {
                     const StockRec st = pf.stocks[i];
                     const double v = simulate_stock_d(st.S0, st.mu, st.sigma, pf.tau, W);
                     Rw[(uint64_t)i * stride] = v;
-                    if (Rw32) Rw32[(uint64_t)i * stride] = (float)v;
+                    if (Rw32) Rw32[(uint64_t)i * stride] = (float)(v / st.S0);
                 }
             }
             acc.st(it.inst, 5, os.nn);
@@ -258,54 +258,58 @@ struct PortfolioPolicyT {
         Kahan b1, b2, bab;
         float mm = 0.f;
         bool redo64 = false;  // a term at a payoff discontinuity (mixed form)
-        if (EXACT_ONLY && F32) {
+        if constexpr (EXACT_ONLY && F32) {
             // Two inner samples per iteration: both option searches and record
             // loads are issued before either sample's Box-Muller block is
             // computed, so one sample's gathers overlap the other's arithmetic.
+            // The FP32 terms are added in FP64.
             const double cp = pf.compute_prob[1];
             const double wc = pf.w_est_const;
-            // The outer sample's stock levels as FP32 (half the bytes of the
-            // FP64 row per gather; the same values the FP64 row rounds to).
-            const float* R32 = A.R32 ? A.R32 + m * rstride(A) : nullptr;
-            auto Rf = [&](uint32_t si) -> float { return R32 ? R32[si] : (float)R[si]; };
+            const bool anti = pf.use_antithetic_risk, cv = pf.use_delta_cv;
+            const float* const Rr = A.R32 + m * rstride(A);  // levels at tau over S0
+            double bm = 0.;
             float m2 = 0.f;
-            auto term = [&](const MixRec& q, float Rq, const u64x2& blk1, uint32_t idx) {
+            auto term = [&](const MixRec& q, float Rq, const u64x2& blk1, uint32_t idx) -> float {
                 float x, y, mag;
                 boxmuller_f32(blk1.a, blk1.b, x, y);  // second = word 3 (element a), first = word 2
-                const MixStock st = pf.mix_stocks[q.stype >> 8];
-                const float d = inner_exact_mix(q, st, pf.use_antithetic_risk, pf.use_delta_cv, Rq, x, y, mag);
-                work += wc >= 0. ? wc : pf.options[1][idx].W_est;
-                b1.add(d);
-                b2.add(d * d);
-                bab.add(mag);
-                m2 += mag * (fabsf(d) + 0x1p-19f * mag);
+                const float d = inner_exact_mix(q, pf.mix_stocks[q.stype >> 8], anti, cv, Rq, x, y, mag);
+                if (wc < 0.) work += pf.options[1][idx].W_est;
+                const double dd = (double)d;
+                a1 += dd;
+                if (TEST) {
+                    a2 = __builtin_fma(dd, dd, a2);
+                    m2 += mag * (fabsf(d) + 0x1p-19f * mag);
+                }
+                return mag;
             };
+            const uint64_t ctag = (uint64_t)tag << 40;
             uint64_t u = u0;
             for (; u + 1 < u1; u += 2) {
-                const uint64_t ca = ((uint64_t)tag << 40) | u, cb = ca + 1;
+                const uint64_t ca = ctag | u, cb = ca + 1;
                 const u64x2 a0 = threefry2x64_20(0, ca, seed, k1);
                 const u64x2 b0 = threefry2x64_20(0, cb, seed, k1);
                 const uint32_t ia = pick_cdf(pf, 1, u01_f64(a0.a) * cp);
                 const uint32_t ib = pick_cdf(pf, 1, u01_f64(b0.a) * cp);
                 const MixRec qa = pf.mix[ia], qb = pf.mix[ib];
-                const float Ra = Rf(qa.stype >> 8), Rb = Rf(qb.stype >> 8);
-                const u64x2 a1 = threefry2x64_20(1, ca, seed, k1);
+                const float Ra = Rr[qa.stype >> 8], Rb = Rr[qb.stype >> 8];
+                const u64x2 a1k = threefry2x64_20(1, ca, seed, k1);
                 const u64x2 b1k = threefry2x64_20(1, cb, seed, k1);
-                term(qa, Ra, a1, ia);
-                term(qb, Rb, b1k, ib);
+                const float ma = term(qa, Ra, a1k, ia);
+                bm += (double)(ma + term(qb, Rb, b1k, ib));
             }
             if (u < u1) {
-                const uint64_t ca = ((uint64_t)tag << 40) | u;
+                const uint64_t ca = ctag | u;
                 const u64x2 a0 = threefry2x64_20(0, ca, seed, k1);
                 const uint32_t ia = pick_cdf(pf, 1, u01_f64(a0.a) * cp);
                 const MixRec qa = pf.mix[ia];
-                term(qa, Rf(qa.stype >> 8), threefry2x64_20(1, ca, seed, k1), ia);
+                bm += (double)term(qa, Rr[qa.stype >> 8], threefry2x64_20(1, ca, seed, k1), ia);
             }
+            if (wc >= 0.) work = wc * (double)(u1 - u0);
             s.nu += 2 * (u1 - u0);
             s.nn += 2 * (u1 - u0);
-            s.s1 += b1.value();
-            s.s2 += b2.value();
-            s.sab += bab.value();
+            s.s1 += a1;
+            s.s2 += a2;
+            s.sab += bm;
             s.smm += m2;
             s.work += work;
             return;
@@ -398,7 +402,7 @@ struct PortfolioPolicyT {
                             const MixRec q = pf.mix[idx];
                             const uint32_t si = q.stype >> 8;
                             d = inner_exact_mix(q, pf.mix_stocks[si], pf.use_antithetic_risk, pf.use_delta_cv,
-                                                (float)R[si], x, y, mag);
+                                                (float)(R[si] * pf.exact_stocks[si].invS0), x, y, mag);
                         } else {
                             bool exact64;
                             const float ip = (float)pf.options_count;
@@ -565,7 +569,7 @@ __global__ __launch_bounds__(64 * kOuterWaves) void k_pf_outer_mfma(typename P::
             if (m < m_end) {
                 const double v = simulate_stock_d(st.S0, st.mu, st.sigma, pf.tau, pf.stau * acc[i]);
                 A.R_tau[m * rs + n] = v;
-                if (A.R32) A.R32[m * rs + n] = (float)v;
+                if (A.R32) A.R32[m * rs + n] = (float)(v / st.S0);
             }
         }
     }

@@ -58,7 +58,8 @@ __global__ __launch_bounds__(256) void k_stage(StageArgs A) {
         const double w = o.w * exp_d(-A.r * o.maturity);
         const double Tt = o.maturity - A.tau, sTt = sqrt(Tt);
         const uint32_t stype = (o.stock_ind << 8) | (uint32_t)(o.type + 2);
-        A.mix[t] = MixRec{(float)o.strike, (float)sTt, (float)(w * A.prob_norm / o.prob), stype};
+        const double S0 = A.stocks[o.stock_ind].S0, h = 0.5 * w * A.prob_norm / o.prob;
+        A.mix[t] = MixRec{(float)(o.strike / S0), (float)sTt, (float)(is_digital(o.type) ? h : h * S0), stype};
         const double discp = A.subsample == 1    ? w / (o.prob / A.prob_norm)
                              : A.subsample == -1 ? w * A.options_count
                                                  : w;
@@ -67,14 +68,9 @@ __global__ __launch_bounds__(256) void k_stage(StageArgs A) {
         if (t >= A.d) return;
         const StockRec st = A.stocks[t];
         const double dcoef = A.r - 0.5 * st.sigma * st.sigma;
-        MixStock q{};
-        q.sig = (float)st.sigma;
-        q.dcoef = (float)dcoef;
-        q.sigtau = (float)(st.sigma * A.stau);
-        q.S0e = (float)(st.S0 * exp_d(dcoef * A.tau));
-        q.S0 = (float)st.S0;
-        q.invS0 = (float)(1. / st.S0);
-        A.ms[t] = q;
+        const double log2e = 0x1.71547652b82fep+0;
+        A.ms[t] = MixStock{(float)(st.sigma * log2e), (float)(dcoef * log2e), (float)(st.sigma * A.stau * log2e),
+                           (float)exp_d(dcoef * A.tau)};
         A.es[t] = ExactStock{st.sigma, dcoef, dcoef * A.tau, A.stau, st.S0, 1. / st.S0};
     }
 }
