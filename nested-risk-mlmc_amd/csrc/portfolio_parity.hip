@@ -89,7 +89,7 @@ enum { PAR_GENERAL = 0, PAR_EXACT = 1, PAR_NO_UNBIASED = 2 };
 //
 // On one lane (63 idle) a sample took some 1500 dependent instructions: the mix of
 // the reference's own main (1000 options, levels 0..3, 8192 outer samples at level 0)
-// 43 ms a sweep, 7.1 ms this way.
+// 43 ms a sweep, 4.2 ms this way.
 struct GeneralScratch {
     static constexpr uint32_t kFlat = 20;    // pairs of a sample of the flat list
     static constexpr uint32_t kPairs = 384;  // the list's buffer
@@ -252,17 +252,21 @@ __device__ __forceinline__ InnerSums general_inner(const PortfolioParityArgs& A,
         double w = si.saved;
         if ((exact || unb) && sb && (before || !wait_known)) {
             double x;
-            stream_bm_f64(A.seed, k1, before ? prev_end - 2 : wait_pos, x, w);
+            stream_bm_any_f64(A.seed, k1, before ? prev_end - 2 : wait_pos, x, w);
         }
         if (mine) {
             nu += unb ? 3 : 2;
             nn += exact ? 2 : unb ? 1 + N : 0;
         }
         uint32_t idx = 0;
-        if (mine) idx = pick_in_method(pf, method, u01_f64(stream_word(A.seed, k1, Pn - 1)));
+        Words3 wd{};
+        if (mine) {
+            wd = stream_words3(A.seed, k1, Pn - 1);
+            idx = pick_in_method(pf, method, u01_f64(wd.w0));
+        }
         if (exact) {
             double x, y;
-            stream_bm_f64(A.seed, k1, Pn, x, y);
+            boxmuller_f64(wd.w2, wd.w1, x, y);
             add(exact_term(pf, idx, R, sb ? w : x, sb ? x : y, work));
         }
         if (bs) {
@@ -293,7 +297,7 @@ __device__ __forceinline__ InnerSums general_inner(const PortfolioParityArgs& A,
                 const int o = c < cnt ? (int)sc.owner[c] : (int)lane;
                 const uint64_t oP = __shfl((unsigned long long)Pn, o, 64);
                 const uint32_t oo = (uint32_t)__shfl((int)off, o, 64) - base;
-                if (c < cnt) stream_bm_f64(A.seed, k1, oP + 2 * (uint64_t)(c - oo), sc.z[2 * c], sc.z[2 * c + 1]);
+                if (c < cnt) stream_bm_any_f64(A.seed, k1, oP + 2 * (uint64_t)(c - oo), sc.z[2 * c], sc.z[2 * c + 1]);
             }
             lds_fence();
             if (sel) {
@@ -364,15 +368,33 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
     const bool fast = pf.subsample != 0 && !(pf.compute_prob[2] > 0) && !si.is_saved;
     if (EXACT_ONLY && fast) {
         // Every option Exact: method 1 for every sample, three inner words each.
+        // A lane takes two consecutive samples, six words: three blocks when the
+        // stream stands at an even word, four at an odd one, and the parity is the
+        // same in all lanes.  (One sample a lane leaves neighbouring lanes at
+        // different parities, which costs four blocks a sample.)
         double s1 = 0., s2 = 0., work = 0.;
-        for (uint64_t k = tid; k < count; k += 64 * W) {
-            const uint64_t q = si.P + 3 * k;
-            const uint32_t idx = pick_in_method(pf, 1, u01_f64(stream_word(A.seed, k1, q)));
+        auto sample = [&](uint64_t w0, uint64_t w1, uint64_t w2) {
+            const uint32_t idx = pick_in_method(pf, 1, u01_f64(w0));
             double x, y;
-            stream_bm_f64(A.seed, k1, q + 1, x, y);
+            boxmuller_f64(w2, w1, x, y);
             const double v = exact_term(pf, idx, R, x, y, work);
             s1 += v;
             s2 += v * v;
+        };
+        const bool odd = si.P & 1;
+        for (uint64_t k = 2 * tid; k < count; k += 128 * W) {
+            const uint64_t b = (si.P + 3 * k) >> 1;
+            const u64x2 b0 = threefry2x64_20(b, 0, A.seed, k1), b1 = threefry2x64_20(b + 1, 0, A.seed, k1),
+                        b2 = threefry2x64_20(b + 2, 0, A.seed, k1);
+            uint64_t v0, v1, v2;
+            if (!odd) {
+                sample(b0.b, b0.a, b1.b);
+                v0 = b1.a, v1 = b2.b, v2 = b2.a;
+            } else {
+                sample(b0.a, b1.b, b1.a);
+                v0 = b2.b, v1 = b2.a, v2 = threefry2x64_20(b + 3, 0, A.seed, k1).b;
+            }
+            if (k + 1 < count) sample(v0, v1, v2);
         }
         const double a = wave_sum(s1), b = wave_sum(s2), c = wave_sum(work);
         if (lane == 0) {
@@ -406,11 +428,12 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
             const uint64_t nvalid = count - c0 < 64 ? count - c0 : 64;
             const uint64_t q = si.P + base + (valid ? lane + 2 * __popcll(exact & below) : 0);
             if (valid) {
-                const uint32_t idx = pick_in_method(pf, method, u01_f64(stream_word(A.seed, k1, q)));
+                const Words3 w = stream_words3(A.seed, k1, q);
+                const uint32_t idx = pick_in_method(pf, method, u01_f64(w.w0));
                 double v;
                 if (method == 1) {
                     double x, y;
-                    stream_bm_f64(A.seed, k1, q + 1, x, y);
+                    boxmuller_f64(w.w2, w.w1, x, y);
                     v = exact_term(pf, idx, R, x, y, work);
                     nn += 2;
                 } else {
@@ -507,16 +530,12 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
     return r;
 }
 
-// Waves per SIMD the kernels are compiled for.  Exact-only, measured on the
-// large and small books' plain sweeps: 2 (what the compiler picks unasked,
-// 235-255 VGPRs, 336 B of scratch a lane) 18.5 and 13.2 ms, 3 (168 VGPRs,
-// 624 B) 17.0 and 12.9 ms, 4 (128 VGPRs, 800 B) 17.4 and 13.0 ms.  The
-// other two, left alone, get the whole register file and one wave a SIMD; at
-// 2 a book of 4000 BS and 6000 Exact options sweeps (levels 0..4) in 24.1
-// against 31.0 ms, one of 3000 BS, 5000 Exact and 2000 Unbiased options in
-// 1.53 against 2.28 s (at 3 the spills make both slower).
+// Waves per SIMD the kernels are compiled for: 2, which leaves the Exact-only
+// kernel's two samples a lane in registers (small book's plain sweep 8.4 ms; at 3,
+// 384 B of scratch a lane, 9.3 ms; at 4, 528 B, 10.0 ms) and the general one's window
+// nearly so (the reference main's mix 5.7 ms; at 3 6.7 ms).
 #ifndef NMLMC_PLAIN_EXACT_WAVES
-#define NMLMC_PLAIN_EXACT_WAVES 3
+#define NMLMC_PLAIN_EXACT_WAVES 2
 #endif
 #ifndef NMLMC_PLAIN_NO_UNBIASED_WAVES
 #define NMLMC_PLAIN_NO_UNBIASED_WAVES 2
@@ -529,7 +548,9 @@ template <uint32_t W, int KIND>
 __global__ __launch_bounds__(64 * W, (KIND == PAR_EXACT ? NMLMC_PLAIN_EXACT_WAVES : KIND == PAR_NO_UNBIASED ? NMLMC_PLAIN_NO_UNBIASED_WAVES : NMLMC_PLAIN_GENERAL_WAVES)) void k_portfolio_parity(
     PortfolioParityArgs A) {
     constexpr bool EXACT_ONLY = KIND == PAR_EXACT;
-    extern __shared__ double smem[];  // R_tau[d], z[d], reduction scratch[kParityRed]
+    // R_tau[d], z[d], reduction scratch[kParityRed], then the moment sums, which
+    // thread 0 keeps (in registers, 32 doubles in every lane, they spilled).
+    extern __shared__ double smem[];
     const PortfolioDevice& pf = A.pf;
     const EngineParams& ep = A.ep;
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
@@ -538,6 +559,10 @@ __global__ __launch_bounds__(64 * W, (KIND == PAR_EXACT ? NMLMC_PLAIN_EXACT_WAVE
     double* R = smem;
     double* z = smem + d;
     double* red = smem + 2 * d;
+    double* f_sums = red + kParityRed;
+    double* d_sums = f_sums + kMaxPhi * kMaxMoments;
+    if (tid == 0)
+        for (int i = 0; i < kMaxPhi * kMaxMoments; i++) f_sums[i] = d_sums[i] = 0.;
 
     uint64_t q = A.M / A.T, rr = A.M % A.T;
     if (t < rr) {
@@ -546,7 +571,6 @@ __global__ __launch_bounds__(64 * W, (KIND == PAR_EXACT ? NMLMC_PLAIN_EXACT_WAVE
     }
     const uint64_t s0 = q * t + rr, e0 = s0 + q;
     StreamState ss = A.states[2 * t], si = A.states[2 * t + 1];
-    double f_sums[kMaxPhi * kMaxMoments] = {}, d_sums[kMaxPhi * kMaxMoments] = {};
     uint64_t stats[kStatsExt] = {0, 0, 0, 0, 0, 0, 0, 0};
     double work = 0.;
     const bool fine_only = A.ell == 0;
@@ -594,79 +618,90 @@ __global__ __launch_bounds__(64 * W, (KIND == PAR_EXACT ? NMLMC_PLAIN_EXACT_WAVE
         if constexpr (!EXACT_ONLY)
             if (pf.subsample == 0) start += det_bs_sum(pf, R, w_det);
 
-        auto test_round = [&](uint64_t cur) {
-            const InnerSums s = parity_inner<W, KIND>(A, R, k1, ss, si, cur, red);
-            work += s.work + A.bs_work;
-            stats[4] += s.nu;
-            stats[5] += s.nn;
-            const double out_var = s.s2 / (double)(cur - 1) - (s.s1 * s.s1) / (double)(cur * (cur - 1));
-            const double dist = start + s.s1 / (double)cur;
-            return dist * dist / out_var;
-        };
-        auto count_of = [&](const LevelCounts& lc, bool with_stats) {
-            uint64_t cur = lc.base;
-            while (true) {
-                if (lc.max <= 2 * cur) {
-                    cur = lc.max;
-                    break;
+        // The outer sample's draw groups one after another, from one call of the
+        // inner loop (inlined at the five places that the reference calls it from,
+        // it outgrew the instruction cache and the registers): the test rounds of
+        // the fine count (phase 0) and of the coarse one (1), then the finals (2).
+        uint64_t nf = 0, nc = 0, cur = A.cf.base;
+        uint64_t group = 0, groups = 1, small = 0, big = 0;
+        bool f_big = true;
+        double f_phi[kMaxPhi] = {}, c_phi[kMaxPhi] = {}, s1_big = 0.;
+        int phase = 0;
+        while (true) {
+            bool decided = false;
+            uint64_t n;
+            if (phase < 2) {
+                const uint64_t lmax = phase == 0 ? A.cf.max : A.cc.max;
+                n = cur;
+                if (lmax <= 2 * cur) {
+                    cur = lmax;
+                    decided = true;
+                } else {
+                    stats[0] += cur;
                 }
-                stats[0] += cur;
-                const double delta2 = test_round(cur);
-                const double nc = (lc.rule == 1) ? lc.tmp / delta2 : pow(delta2, -ep.adaptive_r / 2) * lc.tmp;
-                if (nc <= (double)cur) break;
-                cur *= 2;
-            }
-            if (with_stats) {
-                stats[1] += 1;
-                stats[2] += (cur == lc.max);
-                stats[3] += (cur == lc.base);
-            }
-            return cur;
-        };
-        auto mean_of = [&](uint64_t n) {
-            const InnerSums s = parity_inner<W, KIND>(A, R, k1, ss, si, n, red);
-            work += s.work + A.bs_work;
-            stats[4] += s.nu;
-            stats[5] += s.nn;
-            return s.s1;
-        };
-
-        const uint64_t nf = count_of(A.cf, true);
-        uint64_t nc = 0;
-        double f_phi[kMaxPhi] = {}, c_phi[kMaxPhi] = {};
-        if (fine_only) {
-            stats[0] += nf;
-            phi_add(pf, start + mean_of(nf) / (double)nf, 1., f_phi);
-        } else {
-            nc = count_of(A.cc, false);
-            if (ep.antithetic) {
-                const bool f_big = nf > nc;
-                const uint64_t big = f_big ? nf : nc, small = f_big ? nc : nf;
-                const uint64_t groups = big / small;
-                const double coeff = (double)(1.f / (float)groups);
-                double s1_big = 0.;
-                double* out_small = f_big ? c_phi : f_phi;
-                double* out_big = f_big ? f_phi : c_phi;
-                for (uint64_t g = 0; g < groups; g++) {
-                    const double s1 = mean_of(small);
-                    phi_add(pf, start + s1 / (double)small, coeff, out_small);
-                    s1_big += s1;
-                }
-                phi_add(pf, start + s1_big / (double)big, 1., out_big);
-                stats[0] += big;
             } else {
-                stats[0] += nf + nc;
-                phi_add(pf, start + mean_of(nf) / (double)nf, 1., f_phi);
-                phi_add(pf, start + mean_of(nc) / (double)nc, 1., c_phi);
+                n = (fine_only || ep.antithetic) ? small : group == 0 ? nf : nc;
+            }
+            if (!decided) {
+                const InnerSums s = parity_inner<W, KIND>(A, R, k1, ss, si, n, red);
+                work += s.work + A.bs_work;
+                stats[4] += s.nu;
+                stats[5] += s.nn;
+                if (phase < 2) {
+                    const double tmp = phase == 0 ? A.cf.tmp : A.cc.tmp;
+                    const double out_var = s.s2 / (double)(n - 1) - (s.s1 * s.s1) / (double)(n * (n - 1));
+                    const double dist = start + s.s1 / (double)n;
+                    const double delta2 = dist * dist / out_var;
+                    const double want = A.cf.rule == 1 ? tmp / delta2 : pow(delta2, -ep.adaptive_r / 2) * tmp;
+                    if (want <= (double)n) decided = true;
+                    else cur *= 2;
+                } else if (fine_only) {
+                    phi_add(pf, start + s.s1 / (double)nf, 1., f_phi);
+                } else if (ep.antithetic) {
+                    const double coeff = (double)(1.f / (float)groups);
+                    phi_add(pf, start + s.s1 / (double)small, coeff, f_big ? c_phi : f_phi);
+                    s1_big += s.s1;
+                } else {
+                    phi_add(pf, start + s.s1 / (double)n, 1., group == 0 ? f_phi : c_phi);
+                }
+                if (phase == 2 && ++group == groups) break;
+            }
+            if (!decided) continue;
+            if (phase == 0) {
+                nf = cur;
+                stats[1] += 1;
+                stats[2] += (nf == A.cf.max);
+                stats[3] += (nf == A.cf.base);
+                cur = A.cc.base;
+                phase = fine_only ? 2 : 1;
+            } else {
+                nc = cur;
+                phase = 2;
+            }
+            if (phase == 2) {
+                if (fine_only) {
+                    small = nf;
+                    stats[0] += nf;
+                } else if (ep.antithetic) {
+                    f_big = nf > nc;
+                    big = f_big ? nf : nc;
+                    small = f_big ? nc : nf;
+                    groups = big / small;
+                    stats[0] += big;
+                } else {
+                    groups = 2;
+                    stats[0] += nf + nc;
+                }
             }
         }
-        add_moments(f_phi, ps, f_sums, ep.fine_moments);
-        if (!fine_only) {
-            double dphi[kMaxPhi];
-            for (uint32_t i = 0; i < ps; i++) dphi[i] = f_phi[i] - c_phi[i];
-            add_moments(dphi, ps, d_sums, ep.diff_moments);
-        }
+        if (!fine_only && ep.antithetic) phi_add(pf, start + s1_big / (double)big, 1., f_big ? f_phi : c_phi);
         if (tid == 0) {
+            add_moments(f_phi, ps, f_sums, ep.fine_moments);
+            if (!fine_only) {
+                double dphi[kMaxPhi];
+                for (uint32_t i = 0; i < ps; i++) dphi[i] = f_phi[i] - c_phi[i];
+                add_moments(dphi, ps, d_sums, ep.diff_moments);
+            }
             if (A.tr_phi_f) A.tr_phi_f[m] = f_phi[0];
             if (A.tr_phi_c) A.tr_phi_c[m] = fine_only ? 0. : c_phi[0];
             if (A.tr_nf) A.tr_nf[m] = nf;
@@ -707,9 +742,8 @@ hipError_t launch_portfolio_parity(const PortfolioParityHost& H, hipStream_t s) 
     // Waves per virtual thread: more than one only for books whose options are
     // all Exact, while the virtual threads with outer samples (min(M, T)) are
     // too few to fill the device: up to kMaxW, doubling while they stay within
-    // a budget of 6144 waves (the Exact-only kernel runs three waves a SIMD;
-    // the large and small books' plain sweeps took 16.9 and 12.5 ms at a
-    // budget of 1536, 16.3 and 11.7 ms at 6144, 16.5 and 11.5 ms at 12288).
+    // a budget of 6144 waves (the small book's plain sweep takes 9.8 ms at a budget
+    // of 1024, 8.8 at 2048, 8.6 at 6144 and 8.6 at 12288).
     // NMLMC_PLAIN_WAVE_BUDGET and NMLMC_PLAIN_WAVES (1, 2, 4 or 8) override it;
     // per-sample results do not depend on it.
     uint32_t W = 1;
@@ -726,7 +760,7 @@ hipError_t launch_portfolio_parity(const PortfolioParityHost& H, hipStream_t s) 
             W = (v >= 8) ? 8 : (v >= 4) ? 4 : (v >= 2) ? 2 : 1;
         }
     }
-    const size_t lds = sizeof(double) * (2 * (size_t)H.pf.d + kParityRed);
+    const size_t lds = sizeof(double) * (2 * (size_t)H.pf.d + kParityRed + 2 * kMaxPhi * kMaxMoments);
     switch (W) {
     case 8: hipLaunchKernelGGL((k_portfolio_parity<8, PAR_EXACT>), dim3(H.blocks), dim3(512), lds, s, A); break;
     case 4: hipLaunchKernelGGL((k_portfolio_parity<4, PAR_EXACT>), dim3(H.blocks), dim3(256), lds, s, A); break;

@@ -244,6 +244,22 @@ __device__ __forceinline__ void stream_bm_f64(uint64_t k0, uint64_t k1, uint64_t
     boxmuller_f64(second, first, x, y);
 }
 
+// Words q, q + 1, q + 2 of a stream, and the Box-Muller pair of words P, P + 1,
+// where the lanes of a wave stand at positions of either parity: always two
+// blocks and a select (the branches on the parity would both be taken, three
+// blocks a pair and four with a word before it).
+struct Words3 {
+    uint64_t w0, w1, w2;
+};
+__device__ __forceinline__ Words3 stream_words3(uint64_t k0, uint64_t k1, uint64_t q) {
+    const u64x2 b0 = threefry2x64_20(q >> 1, 0, k0, k1), b1 = threefry2x64_20((q >> 1) + 1, 0, k0, k1);
+    return (q & 1) ? Words3{b0.a, b1.b, b1.a} : Words3{b0.b, b0.a, b1.b};
+}
+__device__ __forceinline__ void stream_bm_any_f64(uint64_t k0, uint64_t k1, uint64_t P, double& x, double& y) {
+    const u64x2 b0 = threefry2x64_20(P >> 1, 0, k0, k1), b1 = threefry2x64_20((P + 1) >> 1, 0, k0, k1);
+    boxmuller_f64((P & 1) ? b1.b : b0.a, (P & 1) ? b0.a : b0.b, x, y);
+}
+
 // A random_state (par_omp.hpp:72-121) positioned on a keyed counter sequence:
 // block b of the stream is threefry({b, c1}, {k0, k1}); word q is element
 // 1 - (q & 1) of block q >> 1.  c1 = 0 for the reference keying's per-thread
