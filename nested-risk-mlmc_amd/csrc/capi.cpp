@@ -119,6 +119,8 @@ void Engine::free_samplers() {
     if (d_states) hipFree(d_states);
     if (d_partials) hipFree(d_partials);
     if (d_ws) hipFree(d_ws);
+    if (d_help) hipFree(d_help);
+    d_help = nullptr;
     d_states = nullptr;
     d_partials = nullptr;
     d_ws = nullptr;
@@ -164,6 +166,24 @@ int Engine::ensure_partials(size_t n) {
     if (e != hipSuccess) return hip_fail(e, "hipMalloc partials");
     partial_cap = n;
     return NMLMC_OK;
+}
+
+// The postings of the plain model calls, cleared once: a call leaves none open, and
+// its counts go on from the last call's.  nullptr (no help) if there is no room.
+PlainHelp* Engine::ensure_help() {
+    if (d_help) return d_help;
+    if (hipMalloc(&d_help, sizeof(PlainHelp)) != hipSuccess) {
+        hipGetLastError();
+        d_help = nullptr;
+        return nullptr;
+    }
+    if (hipMemsetAsync(d_help, 0, offsetof(PlainHelp, sums), stream) != hipSuccess) {
+        hipGetLastError();
+        hipFree(d_help);
+        d_help = nullptr;
+    }
+    help_base = 0;
+    return d_help;
 }
 
 int Engine::ensure_ws(size_t n) {
@@ -317,26 +337,47 @@ int Engine::sample_model_parity(uint32_t ell, uint64_t M, uint32_t lanes_overrid
     H.ell = ell;
     const int nps = mp.variant == MODEL_REF ? 2 : 1;
     const uint64_t pairs = (H.cf.base * nps + 1) / 2;
-    // Lanes per virtual thread: the next power of two of the base count's
-    // Box-Muller pairs, at most a wave; a whole block of 256 lanes when at most
+    // Lanes per virtual thread: a whole block of 256 when at most
     // plain_wide_max() virtual threads hold outer samples and the pairs fill
     // it (the deep levels, whose few outer samples each take up to 2^cap times
-    // the base count on one virtual thread) and the partial records fit.
+    // the base count on one virtual thread) and the partial records fit; else at
+    // most a wave, and no more lanes than the base count's pairs, or than give a
+    // lane kLanePairs pairs of the largest count, unless the lanes in flight would
+    // fall below kLanesFull.  Every lane draws the outer sample and takes part
+    // in the sums, so fewer lanes are less work; too few leave the longest
+    // outer samples of the call on their own.  Reference model, 65536 virtual
+    // threads, r = 1.5, by lanes 1 / 4 / 16 / 64 / 256 (ms): level 0 0.62 / 0.66 / 0.99 / 2.54 /
+    // 11.7 (the base count's pairs alone gave 32: 1.37), level 1 0.81 / 0.83 / 1.10 /
+    // 2.67 / 12.1 (64), level 2 1.54 / 1.49 / 1.52 / 1.79 / 5.45, level 3 5.9 / 2.9 / 2.2 / 1.58 /
+    // 2.98, level 4 19.6 / 6.3 / 2.9 / 1.54 / 1.61, level 5 110 / 21 / 4.3 / 1.63 / 1.09.
+    constexpr uint64_t kLanePairs = 32, kLanesFull = 262144;
+    const uint64_t act = plain_active(M, cores);
+    uint64_t records = 0;
     uint64_t want = lanes_override;
     if (const char* s = getenv("NMLMC_GROUP_LANES")) want = strtoul(s, nullptr, 10);
     if (want) {
         H.G = want >= 256 ? 256 : pow2_ceil_u32(want);
     } else {
-        H.G = pow2_ceil_u32(pairs);
-        const uint64_t act = plain_active(M, cores);
+        const uint64_t most = (H.cf.max * nps + 1) / 2;
+        const uint64_t lanes = std::max(most / kLanePairs, kLanesFull / act);
+        H.G = pow2_ceil_u32(std::max<uint64_t>(1, std::min(pairs, lanes)));
+        // What a caller's scratch must hold does not depend on the lanes chosen here.
+        records = parity_blocks(act, pow2_ceil_u32(pairs));
         if (pairs >= 256 && act <= plain_wide_max() && (!scr_partials || parity_blocks(act, 256) <= scr_cap))
-            H.G = 256;
+            H.G = 256, records = 0;
     }
     last_G = H.G;
-    const uint64_t nblocks = parity_blocks(plain_active(M, cores), H.G);
+    const uint64_t nblocks = parity_blocks(act, H.G);
+    // Blocks help each other where a draw group can be long enough to be posted and
+    // every block has a slot; never in a call that may not allocate.
+    const uint64_t longest = std::max(H.cf.max, H.cc.max) * nps / 2;
+    if (H.G == 256 && longest >= kPostPairs && act <= kHelpSlots && !scr_partials) {
+        H.help = ensure_help();
+        H.help_base = help_base;
+    }
     H.blocks = (uint32_t)nblocks;
     Partial *parts, *res;
-    int rc = plain_buffers(nblocks, parts, res);
+    int rc = plain_buffers(std::max(nblocks, records), parts, res);
     if (rc) return rc;
     H.states = d_states;
     H.partials = parts;
@@ -351,6 +392,7 @@ int Engine::sample_model_parity(uint32_t ell, uint64_t M, uint32_t lanes_overrid
     if (e != hipSuccess) return hip_fail(e, "hipEventRecord");
     e = launch_model_parity(H, stream);
     if (e != hipSuccess) return hip_fail(e, "launch k_model_parity");
+    if (H.help) help_base += H.blocks;
     if ((e = hipEventRecord(ev1, stream)) != hipSuccess) return hip_fail(e, "hipEventRecord");
     e = launch_reduce_partials(parts, (uint32_t)nblocks, res, stream);
     if (e != hipSuccess) return hip_fail(e, "launch k_reduce_partials");

@@ -45,32 +45,74 @@ struct EngineParams {
 
 enum { PHI_INDICATOR = 0, PHI_MAX = 1, PHI_MOMENTS = 2, PHI_FMOMENTS = 3 };
 
-// Sum over the G lanes of an aligned lane group with an xor butterfly: every
-// lane of the group ends with the same, bit-identical, total.
-template <int G>
-__device__ __forceinline__ double group_sum(double v) {
-#pragma unroll
-    for (int o = G / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// One step of a butterfly over aligned groups of lanes: v plus the value O lanes
+// across (lane ^ O), by register moves (DPP, gfx950's row swaps) instead of the
+// LDS permute that a shuffle is: a wave's FP64 sum in a fraction of the latency.
+// DPP has no lane ^ 4 and, upward, no lane ^ 8: a mirror of 8 or 16 lanes where the
+// steps go up (the smaller groups' lanes are equal already), a rotation by 4
+// where they go down (lanes 8 apart are).
+template <int O, bool UP>
+__device__ __forceinline__ uint32_t lane_across(uint32_t v) {
+    static_assert(O == 1 || O == 2 || O == 4 || O == 8, "within a row of 16 lanes");
+    constexpr int quad = O == 1 ? 0xB1 : 0x4E, mirror = O == 4 ? 0x141 : 0x140, rotate = O == 4 ? 0x124 : 0x128;
+    constexpr int ctrl = O <= 2 ? quad : UP ? mirror : rotate;
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, ctrl, 0xf, 0xf, false);
 }
-template <int G>
-__device__ __forceinline__ uint64_t group_sum_u64(uint64_t v) {
+template <int O, bool UP = true, class T>
+__device__ __forceinline__ T add_across(T v) {
+    static_assert(sizeof(T) == 8, "64-bit sums");
+    uint32_t w[2], a[2], b[2];
+    __builtin_memcpy(w, &v, 8);
 #pragma unroll
-    for (int o = G / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    for (int i = 0; i < 2; i++) {
+        if constexpr (O < 16) {
+            a[i] = w[i];
+            b[i] = lane_across<O, UP>(w[i]);
+        } else if constexpr (O == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(w[i], w[i], false, false);
+            a[i] = r[0];
+            b[i] = r[1];
+        } else {
+            const auto r = __builtin_amdgcn_permlane32_swap(w[i], w[i], false, false);
+            a[i] = r[0];
+            b[i] = r[1];
+        }
+    }
+    T x, y;
+    __builtin_memcpy(&x, a, 8);
+    __builtin_memcpy(&y, b, 8);
+    return x + y;
 }
 
-// Sum of a double over the 64 lanes of a wave.
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+// Sum over the G lanes of an aligned lane group: every lane of the group ends
+// with the same, bit-identical, total.
+template <int G, class T>
+__device__ __forceinline__ T group_total(T v) {
+    if constexpr (G > 1) v = add_across<1>(v);
+    if constexpr (G > 2) v = add_across<2>(v);
+    if constexpr (G > 4) v = add_across<4>(v);
+    if constexpr (G > 8) v = add_across<8>(v);
+    if constexpr (G > 16) v = add_across<16>(v);
+    if constexpr (G > 32) v = add_across<32>(v);
     return v;
 }
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+    return group_total<G>(v);
 }
+
+// Sums over the 64 lanes of a wave, halves first.
+template <class T>
+__device__ __forceinline__ T wave_total(T v) {
+    v = add_across<32, false>(v);
+    v = add_across<16, false>(v);
+    v = add_across<8, false>(v);
+    v = add_across<4, false>(v);
+    v = add_across<2, false>(v);
+    return add_across<1, false>(v);
+}
+__device__ __forceinline__ double wave_sum(double v) { return wave_total(v); }
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) { return wave_total(v); }
 
 // Lane `lane`'s value for every lane (lane the same in all lanes; it need not
 // be active for the read, but its value is only meaningful when it is).
@@ -83,48 +125,6 @@ __device__ __forceinline__ uint64_t bcast_u64(uint64_t v, uint32_t lane) {
 }
 __device__ __forceinline__ double bcast_f64(double v, uint32_t lane) {
     return __longlong_as_double((long long)bcast_u64((uint64_t)__double_as_longlong(v), lane));
-}
-
-// Reduces the group-uniform accumulators of a 256-thread block into one
-// Partial record (only group leaders contribute).  Every thread of the block
-// must call it.
-__device__ __forceinline__ void block_write_partial(bool leader, const double* f, uint32_t nf,
-                                                    const double* d, uint32_t nd, double work,
-                                                    const uint64_t* st, Partial* out) {
-    __shared__ double sd[4];
-    __shared__ uint64_t su[4];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int k = 0; k < kPartialFields; k++) {
-        const bool is_u = k >= 2 * kMaxPhi * kMaxMoments + 1;
-        double v = 0.;
-        uint64_t u = 0;
-        if (leader) {
-            if (k < kMaxPhi * kMaxMoments) v = (uint32_t)k < nf ? f[k] : 0.;
-            else if (k < 2 * kMaxPhi * kMaxMoments) {
-                const int j = k - kMaxPhi * kMaxMoments;
-                v = (uint32_t)j < nd ? d[j] : 0.;
-            } else if (!is_u) v = work;
-            else u = st[k - (2 * kMaxPhi * kMaxMoments + 1)];
-        }
-        if (is_u) {
-            u = wave_sum_u64(u);
-            if (lane == 0) su[wave] = u;
-        } else {
-            v = wave_sum(v);
-            if (lane == 0) sd[wave] = v;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            if (is_u) out->stats[k - (2 * kMaxPhi * kMaxMoments + 1)] = su[0] + su[1] + su[2] + su[3];
-            else {
-                const double t = ((sd[0] + sd[1]) + sd[2]) + sd[3];
-                if (k < kMaxPhi * kMaxMoments) out->f[k] = t;
-                else if (k < 2 * kMaxPhi * kMaxMoments) out->d[k - kMaxPhi * kMaxMoments] = t;
-                else out->work = t;
-            }
-        }
-        __syncthreads();
-    }
 }
 
 // add_moments (nested_sampler.hpp:87-100): out[i*m + j] += phi_i^(j+1).

@@ -62,6 +62,9 @@ struct Engine {
     Partial* h_out = nullptr;
     double* d_ws = nullptr;           // per-group workspace (portfolio R_tau)
     size_t ws_cap = 0;
+    PlainHelp* d_help = nullptr;      // postings of the plain model calls
+    uint32_t help_base = 0;           // its counters: blocks of the calls so far
+    PlainHelp* ensure_help();
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // Scratch of a plain-form level call: the per-block partial records (room

@@ -28,6 +28,30 @@ __device__ __forceinline__ double model_ref_inner(const ModelParams& mp, double 
     return r;
 }
 
+// Helping between the blocks of a plain model call of 256-lane virtual threads.
+// A draw group of kPostPairs Box-Muller pairs or more is posted: its owner and
+// every block that has ended its own virtual thread take segments of it until
+// none is left, and the owner adds the segments' sums in their order, whoever ran
+// them.  Nobody waits for a block that has not started: owners wait only for
+// segments that running blocks hold, and a block that has ended waits for
+// postings only once all blocks have started.
+constexpr uint32_t kPostPairs = 32768, kMinSegment = 8192, kMaxSegments = 256, kHelpSlots = 4096;
+struct alignas(64) PlainJob {  // the block's posting
+    int32_t avail;             // segments not yet taken (0 or less: none)
+    uint32_t finished;
+    uint32_t segment;          // pairs
+    uint32_t pad;
+    uint64_t blk0, pairs, count;
+    double Y;
+};
+struct PlainHelp {
+    alignas(128) uint32_t started;  // blocks, over all calls (wraps)
+    alignas(128) uint32_t ended;
+    alignas(128) uint64_t open[kHelpSlots / 64];  // blocks with a posting; all clear after a call
+    PlainJob job[kHelpSlots];
+    double sums[kHelpSlots][kMaxSegments][2];
+};
+
 struct ModelParityArgsHost {
     ModelParams mp;
     EngineParams ep;
@@ -38,6 +62,8 @@ struct ModelParityArgsHost {
     uint32_t ell;
     uint32_t G;
     uint32_t blocks;  // launched: the blocks of the virtual threads that hold outer samples
+    PlainHelp* help;  // nullptr: blocks do not help each other
+    uint32_t help_base;  // started and ended before the call
     StreamState* states;
     Partial* partials;
     double* tr_phi_f;
