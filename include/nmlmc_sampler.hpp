@@ -225,7 +225,7 @@ int sample(uint32_t ell, uint64_t override_dyn_inner, uint64_t* M, sum_t* fsums,
         A.words = st.words;
         A.obj_words = st.obj_words;
         A.c.phi_type = 0;
-        const Engine::Shape sh = g_engine.batched_shape(ell_eff, *M, 1, A.c, 0);
+        const Engine::Shape sh = g_engine.batched_shape(ell_eff, *M, 1, Engine::ShapeKind::general, A.c, 0);
         A.c.S = sh.S;
         const uint32_t blocks = (uint32_t)g_engine.device_cus() * sh.bpc;
         g_engine.last_kernel = "k_b_final";

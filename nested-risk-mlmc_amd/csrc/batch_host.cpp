@@ -220,6 +220,9 @@ int Engine::batch_sample(uint32_t ell, const uint64_t* Ms, sample_output* outs) 
     H.mixed = form == NMLMC_FORM_MIXED;
     H.exact_only = exact_only;
     H.multi = true;
+    bool coupled = false;
+    for (const BatchInst& b : batch) coupled = coupled || b.pf.coupled;
+    const ShapeKind kind = exact_only ? ShapeKind::exact_book : coupled ? ShapeKind::coupled : ShapeKind::general;
     H.R32 = (H.mixed && H.exact_only) ? pf_R32 : nullptr;
     H.c.phi_type = phi_type;
     H.c.n_inst = n;
@@ -233,7 +236,7 @@ int Engine::batch_sample(uint32_t ell, const uint64_t* Ms, sample_output* outs) 
         H.c.offset = 0;
         H.c.inst_out = d_inst_out + k * per;
         H.bt = tabs[k];
-        const Shape sh = batched_shape(ell, Mk, 1, H.c, 0);
+        const Shape sh = batched_shape(ell, Mk, 1, kind, H.c, 0);
         H.c.S = sh.S;
         H.blocks = (uint32_t)device_cus() * sh.bpc;
         last_G = H.c.S;

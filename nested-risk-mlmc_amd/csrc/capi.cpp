@@ -839,13 +839,28 @@ uint64_t Engine::batched_chunk() {
 
 // Launch shape of a batched level call.  An explicit segment size (the
 // override argument, else NMLMC_SEGMENT) wins; otherwise the shape
-// autotune_level chose for this form and level, else the default: the largest
-// segment of 64, 32 or 16 units that still cuts the outer samples' first draw
-// groups into at least 2^19 segments (two waves per SIMD over 256 CUs), with
-// 8 blocks per CU.  On the adaptive benchmarks this default is within ~3% of
-// the best fixed segment at every level (larger segments pay fewer hand-offs,
-// smaller ones spread the few large groups of the high levels).
-Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, const BatchedCommon& c,
+// autotune_level chose for this form and level, else a default from the
+// inner units `all` of the outer samples' first draw groups.
+//
+// Segment.  Every lane walks its segments serially and every segment costs a
+// hand-off, so a call takes about a S + b all / S: the best S grows as the root
+// of `all`.  S is the power of two below sqrt(all / 2^k) (k: 14, or 15 or 16
+// where a unit costs more or no refinement follows), up to 16, or 32 for the mixed
+// model's cheap units; from 2^19 segments of 32 or 64 units on, those.  Measured
+// over 280 calls (300 to 10^6 outer samples, levels 0 to 10, every form and
+// kind, S from 1 to 64 and 1 to 16 blocks a CU) the rule is 2-6% from the best
+// pair of each; never fewer than 4 or 16 units and always 8 blocks were 15-28%
+// off, 60% for books with Unbiased options.
+// Model calls whose whole first group fits one lane take a segment of it (no pool
+// entries, no hand-offs: level 1 of the non-adaptive sweep 294 -> 183 us).  Coupled
+// paths at few units are long and uneven: at most 2 (2^17 units: 480-720 us, with 4
+// 850-1400).
+//
+// Blocks.  A pass starts all its blocks whether they have work or not (8 a CU:
+// about 4 us a launch), and the FP64 kernels hold two or three a CU at a time: 2 a
+// CU for few units (a call of 1000 mixed samples 174 -> 128 us), 4 up to 2^24, then
+// 8, which balance better (10^7 samples of the model, not adaptive: 1015 -> 915 us).
+Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
                                     uint32_t lanes_override) {
     if (force.S) return force;
     Shape sh;
@@ -853,24 +868,28 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, cons
     if (t != tuned.end()) {
         sh = t->second;
     } else {
-        sh.bpc = 8;
-        const uint64_t group = c.cf.max > 2 * c.cf.base ? c.cf.base : c.cf.max;
+        const bool adaptive = c.cf.max > 2 * c.cf.base, fp64 = form != NMLMC_FORM_MIXED;
+        const uint64_t group = adaptive ? c.cf.base : c.cf.max;
         const uint64_t units = (group + spu - 1) / spu;
         const uint64_t m = std::min(M, batched_chunk());
-        // The largest segment that still gives the grid about two segments a
-        // lane; groups of at least 1024 units (the deep levels) may go down
-        // to 4 units a segment, smaller ones stop at 16 (their hand-offs).
-        // With 4 allowed, a level sweep of the 16-book Asian batch at 2048
-        // outer samples per instance takes 39.3 instead of 45.0 ms (the
-        // autotuner's shapes: 39.1); the batch drivers' calls, with more outer
-        // samples, keep their segments.
-        const uint32_t smin = units >= 1024 ? 4u : 16u;
-        sh.S = smin;
-        for (uint32_t S : {64u, 32u, 16u, 8u})
-            if (S >= smin && m * ((units + S - 1) / S) >= (1ull << 19)) {
-                sh.S = S;
-                break;
-            }
+        const uint64_t all = m * units;
+        int k = 14;
+        if (kind == ShapeKind::model && fp64) k = adaptive ? 16 : 15;
+        else if (kind == ShapeKind::exact_book) k = adaptive ? (fp64 ? 15 : 14) : 16;
+        const uint32_t most = kind == ShapeKind::model && !fp64 ? 32 : 16;
+        sh.S = 1;
+        while (sh.S < most && all >= ((uint64_t)sh.S * sh.S << k)) sh.S *= 2;
+        for (uint32_t S : {32u, 64u})
+            if (m * ((units + S - 1) / S) >= (1ull << 19)) sh.S = std::max(sh.S, S);
+        if (kind == ShapeKind::model) {
+            const bool whole = adaptive ? units <= 16 && all >= (fp64 ? 1ull << 21 : 1ull << 18)
+                                        : units <= 16 || (units <= 32 && m >= 4096) || (units <= 64 && m >= 32768);
+            if (whole) sh.S = std::max(sh.S, pow2_ceil_u32(units));
+        }
+        if (kind == ShapeKind::coupled && all < (1ull << 18)) sh.S = std::min(sh.S, 2u);
+        const bool general = kind == ShapeKind::general || kind == ShapeKind::coupled;
+        const int few = general ? 20 : fp64 ? 22 : 18, many = general ? 22 : 24;
+        sh.bpc = all < (1ull << few) ? 2 : all < (1ull << many) ? 4 : 8;
     }
     if (lanes_override) {
         sh.S = lanes_override;
@@ -962,7 +981,7 @@ int Engine::sample_batched(uint32_t ell, uint64_t M, uint64_t outer_offset, uint
     H.c.ups = 0;
     // One unit = one Threefry block + one Box-Muller pair (two samples of the
     // shift model, one of the reference model).
-    const Shape sh = batched_shape(ell, M, mp.variant == MODEL_SHIFT ? 2 : 1, H.c, lanes_override);
+    const Shape sh = batched_shape(ell, M, mp.variant == MODEL_SHIFT ? 2 : 1, ShapeKind::model, H.c, lanes_override);
     H.c.S = sh.S;
     last_G = H.c.S;
     H.blocks = (uint32_t)device_cus() * sh.bpc;

@@ -143,7 +143,12 @@ struct Engine {
     // now on (nmlmc_set_level_coupled_paths).
     bool level_coupled = false;
     Shape force{};                    // the candidate autotune_level is timing
-    Shape batched_shape(uint32_t ell, uint64_t M, uint64_t spu, const BatchedCommon& c, uint32_t lanes_override);
+    // What a call's inner samples are: the shift or reference model's, a book's
+    // of Exact options only, another book's or a sampler class's, or those of a
+    // book on level-coupled paths.
+    enum class ShapeKind { model, exact_book, general, coupled };
+    Shape batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
+                        uint32_t lanes_override);
     int autotune_level(uint32_t ell, uint64_t M, Shape& best, double& best_ms);
     // The candidate loop of the autotuners: run(ms) makes one level call at
     // the forced shape and reports its kernel time.

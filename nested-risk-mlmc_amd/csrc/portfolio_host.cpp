@@ -345,7 +345,11 @@ int Engine::sample_portfolio_batched(uint32_t ell, uint64_t M, uint64_t outer_of
     if (rc) return rc;
     H.pf = pf;
     H.c.phi_type = pf.phi_type;
-    const Shape sh = batched_shape(ell, M, 1, H.c, lanes_override);
+    H.exact_only = pf.subsample == 1 && pf.nopt[0] == 0 && pf.nopt[2] == 0;
+    const ShapeKind kind = H.exact_only ? ShapeKind::exact_book
+                           : pf.coupled ? ShapeKind::coupled
+                                        : ShapeKind::general;
+    const Shape sh = batched_shape(ell, M, 1, kind, H.c, lanes_override);
     H.c.S = sh.S;
     last_G = H.c.S;
     if ((rc = ensure_pf_R(std::min(M, batched_chunk())))) return rc;
@@ -353,7 +357,6 @@ int Engine::sample_portfolio_batched(uint32_t ell, uint64_t M, uint64_t outer_of
     H.bs_work = pf_bs_work;
     H.blocks = (uint32_t)device_cus() * sh.bpc;
     H.mixed = form == NMLMC_FORM_MIXED;
-    H.exact_only = pf.subsample == 1 && pf.nopt[0] == 0 && pf.nopt[2] == 0;
     H.multi = false;
     H.R32 = (H.mixed && H.exact_only) ? pf_R32 : nullptr;
     last_kernel = "k_b_final";
