@@ -122,8 +122,9 @@ __global__ __launch_bounds__(256) void k_b_init(typename P::Args A) {
 // sums may differ from the one the FP64 sums of the same draws give (the
 // batched FP64 form's).  With |s1 - s1_64| <= e1 and |s2 - s2_64| <= e2
 // (P::decision_bounds, plus 2^-21 s2 for the compensated sums' own rounding),
-// |dist - dist_64| <= ed = 2 e1 / n and |var - var_64| <= ev (both doubled to
-// leave room for the FP64 side's rounding), so delta^2_64 lies in
+// |dist - dist_64| <= ed = e1 / n and |var - var_64| <= ev (both a sixteenth larger,
+// which leaves room for the FP64 sums' own rounding, at most n 2^-53 of the terms'
+// magnitudes: a sixteenth of e1 at n = 2^30), so delta^2_64 lies in
 // [qlo, qhi] = [max(|dist| - ed, 0)^2 / (var + ev), (|dist| + ed)^2 / (var - ev)]
 // and the FP64 count new_64 (decreasing in delta^2, as its power -1 or -r/2)
 // in [nlo, nhi]: the decision is uncertain when that interval straddles cur.
@@ -134,7 +135,10 @@ __global__ __launch_bounds__(256) void k_b_init(typename P::Args A) {
 // both bounds are under a tenth of dist and var, delta^2_64 is within 40% of
 // delta^2 and new_64 within a factor 1.7 of new (r < 2), so a decision with
 // new at least a factor 2 from cur is certain without the interval.  The
-// uncertain ones go to the FP64 recheck (k_b_test with RECHECK).
+// uncertain ones go to the FP64 recheck (k_b_test with RECHECK).  With both bounds
+// doubled, and the model's e1 the wider one of its finals, the rechecks took 11% of
+// an MLMC run on the small book; a run takes 60.5 instead of 62.4 ms, the large
+// book's sweep 7.0 instead of 7.15 ms.
 template <class P, int RULE>
 __device__ __forceinline__ bool decision_uncertain(const BatchedCommon& c, const LevelCounts& lc, double start,
                                                    uint64_t cur, double s1, double s2, double sab, double smm) {
@@ -145,8 +149,8 @@ __device__ __forceinline__ bool decision_uncertain(const BatchedCommon& c, const
     const double var = s2 / (n - 1.) - (s1 * s1) / (n * (n - 1.));
     const double dist = start + s1 / n;
     const double ad = fabs(dist);
-    const double ed = 2. * e1 / n;
-    const double ev = 2. * (e2 + (2. * fabs(s1) + e1) * e1 / n) / (n - 1.);
+    const double ed = 1.0625 * e1 / n;
+    const double ev = 1.0625 * (e2 + (2. * fabs(s1) + e1) * e1 / n) / (n - 1.);
     if (!(ed < INFINITY) || !(ev < 0.5 * var)) return true;  // also NaN bounds and var <= 0
     if (ed < 0.1 * ad && ev < 0.1 * var) {
         const double q = dist * dist / var;

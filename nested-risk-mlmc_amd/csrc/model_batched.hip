@@ -43,10 +43,10 @@ struct ModelPolicy {
     // the FP64 sums of the same draws.  Each FP32 term is within
     // e_i = 2^-19 (mag_i + 1) of its FP64 value (normals within 2^-20.5, float
     // rounding of Y and of the products 2^-23 of mag), so |s1 - s1_64| is at
-    // most 2^-19 (sab + n), inside the threshold bound plus 2^-19 n, and
-    // |s2 - s2_64| <= sum(2 |d_i| e_i + e_i^2) with |d_i| <= mag_i.
-    __device__ static void decision_bounds(double n, double start, double sab, double smm, double& e1, double& e2) {
-        e1 = n * mixed_bound(sab / n, start) + 0x1p-19 * n;
+    // most 2^-19 (sab + n) and |s2 - s2_64| <= sum(2 |d_i| e_i + e_i^2) with
+    // |d_i| <= mag_i.
+    __device__ static void decision_bounds(double n, double, double sab, double smm, double& e1, double& e2) {
+        e1 = 0x1p-19 * (sab + n);
         e2 = 0x1p-17 * (smm + sab) + 0x1p-36 * n;
     }
 
