@@ -551,22 +551,28 @@ __global__ __launch_bounds__(256) void k_b_redo_split(typename P::Args A) {
     // serialise on its L2 channel).
     __shared__ double gsum[kRedoGroups];
     const uint32_t n = aload_u32(&c.ctl->nreeval);
-    // Blocks per listed outer sample: one per blockDim.x units of the level's
-    // largest final (its fine or coarse count cap), at most kRedoParts.  The
-    // grid's blocks are dealt out that many to a sample, so that the low
-    // levels' small finals (thousands of listed samples) run side by side and
-    // the high levels' large ones (a few samples of up to 10^6 inner samples)
-    // split wide.  Every block computes the same count; the completing block
-    // waits for exactly these.
+    const uint32_t n_split = n < kRedoSlots ? n : kRedoSlots;
+    if (n_split == 0) return;
+    // Blocks per listed outer sample: the grid over the listed samples, four times
+    // over (their counts differ), but at most one per blockDim.x units of the
+    // level's largest final (its fine or coarse count cap) and at most
+    // kRedoParts.  The few large samples of the high levels (up to 10^6 inner
+    // samples) are so split wide; where a thousand are listed, a lane takes several
+    // units for a block's set-up, sums and ticket: 1448 samples of up to 32768 units 1265 us
+    // with a unit a lane (and a division a unit), 770 now.
+    // Every block computes the same count; the completing block waits for
+    // exactly these.
     const uint64_t cmax = c.cf.max > c.cc.max ? c.cf.max : c.cc.max;
-    const uint64_t want = ((cmax + P::spu - 1) / P::spu + blockDim.x - 1) / blockDim.x;
-    const uint64_t cap = (uint64_t)gridDim.x * gridDim.y < kRedoParts ? (uint64_t)gridDim.x * gridDim.y : kRedoParts;
+    const uint64_t blocks = (uint64_t)gridDim.x * gridDim.y;
+    uint64_t want = ((cmax + P::spu - 1) / P::spu + blockDim.x - 1) / blockDim.x;
+    const uint64_t share = 4 * blocks / n_split;
+    want = want < share ? want : share;
+    const uint64_t cap = blocks < kRedoParts ? blocks : kRedoParts;
     const uint32_t parts = (uint32_t)(want < cap ? (want ? want : 1) : cap);
     const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
     const uint32_t cols = (gridDim.x * gridDim.y) / parts;
     if (b >= cols * parts) return;
     const uint32_t col = b / parts, part = b % parts;
-    const uint32_t n_split = n < kRedoSlots ? n : kRedoSlots;
     for (uint32_t w = col; w < n_split; w += cols) {
         const uint32_t m = c.reeval[w];
         const ItemState& it = c.items[m];
@@ -578,20 +584,21 @@ __global__ __launch_bounds__(256) void k_b_redo_split(typename P::Args A) {
         for (uint32_t g = threadIdx.x; g < kRedoGroups; g += blockDim.x) gsum[g] = 0.;
         __syncthreads();
         double cur = 0.;
-        uint32_t cur_g = ~0u;
-        for (uint64_t k = p0 + threadIdx.x; k < p1; k += blockDim.x) {
-            const uint32_t g = (uint32_t)(k / gu);
-            if (g != cur_g) {
-                if (cur_g != ~0u) atomicAdd(&gsum[cur_g], cur);
+        uint64_t k = p0 + threadIdx.x;
+        uint32_t g = ~0u;
+        for (uint64_t ge = 0; k < p1; k += blockDim.x) {
+            if (k >= ge) {  // a division a group, not one a unit
+                if (g != ~0u) atomicAdd(&gsum[g], cur);
                 cur = 0.;
-                cur_g = g;
+                g = (uint32_t)(k / gu);
+                ge = ((uint64_t)g + 1) * gu;
             }
             SegAcc s;
             const uint64_t i0 = (uint64_t)g * sh.n;
             P::template units<false, false>(A, m, it, TAG_FINAL, k, k + 1, i0, i0 + sh.n, s);
             cur += s.s1;
         }
-        if (cur_g != ~0u) atomicAdd(&gsum[cur_g], cur);
+        if (g != ~0u) atomicAdd(&gsum[g], cur);
         __syncthreads();
         if (p1 > p0) {
             const uint32_t g_lo = (uint32_t)(p0 / gu), g_hi = (uint32_t)((p1 - 1) / gu);
