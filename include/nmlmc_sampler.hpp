@@ -86,6 +86,7 @@ struct SamplerPolicy {
     static constexpr uint64_t spu = 1;
     static constexpr bool kMulti = false;
     static constexpr bool kFuse = true;
+    static constexpr bool kBlock = false;
     static constexpr bool kMixedWaves = false;
     static constexpr bool kTwoValued = false;
 

@@ -403,6 +403,7 @@ struct BatchedCommon {
     uint32_t fcap;
     uint32_t* reeval;
     uint32_t* pend;      // [M] outer samples the fused first pass leaves to the final phase
+    uint32_t block;      // 1: the call is k_b_block's (Engine::block_call)
     uint32_t fused;      // 1: k_b_fused ran (round-0 tests in-lane; final phase over pend)
     double* redo_acc;    // [kRedoSlots x kRedoGroups] FP64 group sums of the redo
     uint32_t* redo_cnt;  // [kRedoSlots] parts of the redo done

@@ -7,6 +7,9 @@
 //   last block lays the final pool out), k_b_final_fill, k_b_final, [k_b_redo_split and
 //   k_b_redo_seq when MIXED]
 #pragma once
+#include <algorithm>
+#include <type_traits>
+
 #include "batched.hpp"
 
 namespace nmlmc {
@@ -1004,6 +1007,185 @@ __global__ __launch_bounds__(256, (mixed_waves<P, MIXED>())) void k_b_fused(type
     acc.template flush<true>(c);
 }
 
+// Sums of the block's 256 threads, in every thread; all of them must call it.
+template <int N>
+__device__ __forceinline__ void block_sums(double (&v)[N]) {
+    __shared__ double part[N][4];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const double w = wave_sum(v[i]);
+        if ((threadIdx.x & 63) == 0) part[i][threadIdx.x >> 6] = w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = ((part[i][0] + part[i][1]) + part[i][2]) + part[i][3];
+    __syncthreads();
+}
+
+// The block's run of units [0, U) of a draw group, lane by lane.
+__device__ __forceinline__ void lane_run(uint64_t U, uint64_t& k0, uint64_t& k1) {
+    const uint64_t run = (U + blockDim.x - 1) / blockDim.x;
+    k0 = threadIdx.x * run;
+    k1 = k0 + run < U ? k0 + run : U;
+}
+
+// Small level calls in one launch: a block takes an outer sample from its draw
+// to its moments, its lanes sharing the inner samples of every round and of
+// the final, and the FP64 recheck and redo of a mixed sample follow in place.
+// Draws, decisions and counts are those of the launch sequence.  For antithetic
+// finals (or level 0) of at most kRedoGroups groups whose sizes are whole units.
+//
+// Bound by latency: of a lane's run of inner samples, round after round, and of the
+// block's sums.  The sequence spends 5 to 17 launches on such a call, 2 to 15 us each
+// whether there is work or not: a call of 1000 mixed model samples at level 3 takes 78 us
+// here and 134 there, 300 of a book at level 0 72 and 172 (Engine::block_call has
+// the lines).  More blocks than fit at a time: a long sample holds back its own only.
+constexpr uint32_t kBlockGrid = 4096;
+template <class P, bool MIXED, int RULE>
+__global__ __launch_bounds__(256, 4) void k_b_block(typename P::Args A) {
+    const BatchedCommon& c = A.c;
+    BlockAcc<P::kMulti> acc;
+    acc.template init<true>(c);
+    __shared__ ItemState it;
+    __shared__ double gs[kRedoGroups], gab[kRedoGroups];
+    __shared__ uint32_t redo;
+    const bool first = threadIdx.x == 0;
+    for (uint64_t m = blockIdx.x; m < c.M; m += gridDim.x) {
+        if (first) {
+            ItemState t;
+            P::init_item(A, m, t, acc);
+            t.nf = t.nc = 0;
+            it = t;
+        }
+        __syncthreads();  // and the outer states that init_item wrote
+        const uint32_t q = it.inst;
+        const double start = it.start;
+        // The refinement rounds of the fine count, then of the coarse one.
+        for (int side = 0; side < (c.ell > 0 ? 2 : 1); side++) {
+            const bool fine = side == 0;
+            const LevelCounts& lc = fine ? c.cf : c.cc;
+            uint64_t n = lc.max;
+            if (lc.max > 2 * lc.base) {
+                n = lc.base;
+                if (first) acc.st(q, 0, n);
+                bool more = true;
+                for (uint32_t r = 0; more; r++) {
+                    const uint64_t cur = n;
+                    const uint32_t tag = (fine ? TAG_FINE_TEST : TAG_COARSE_TEST) + r;
+                    uint64_t k0, k1;
+                    lane_run((cur + P::spu - 1) / P::spu, k0, k1);
+                    SegAcc s;
+                    if (k0 < k1) P::template units<MIXED, true>(A, (uint32_t)m, it, tag, k0, k1, 0, cur, s);
+                    acc.work(q, s.work);
+                    acc.st(q, 4, s.nu);
+                    acc.st(q, 5, s.nn);
+                    if (first) acc.work(q, P::group_work(A, it));
+                    double v[4] = {s.s1, s.s2, s.sab, s.smm};
+                    block_sums(v);
+                    if (MIXED && decision_uncertain<P, RULE>(c, lc, start, cur, v[0], v[1], v[2], v[3])) {
+                        if (first) acc.st(q, 8, 1);
+                        SegAcc d;
+                        if (k0 < k1) P::template units<false, true>(A, (uint32_t)m, it, tag, k0, k1, 0, cur, d);
+                        v[0] = d.s1;
+                        v[1] = d.s2;
+                        block_sums(v);
+                    }
+                    n = next_count<RULE>(c, lc, start, cur, v[0], v[1], more);
+                    if (first && more) acc.st(q, 0, n);
+                }
+            }
+            if (first) {
+                if (fine) {
+                    it.nf = n;
+                    acc.st(q, 1, 1);
+                    acc.st(q, 2, n == lc.max);
+                    acc.st(q, 3, n == lc.base);
+                } else {
+                    it.nc = n;
+                }
+            }
+        }
+        __syncthreads();
+        const FinalShape sh = final_shape(c, it);
+        const uint64_t gu = sh.n / P::spu;
+        uint64_t k0, k1;
+        lane_run(sh.groups * gu, k0, k1);
+        const double coeff = (double)(1.f / (float)sh.groups);
+        double phi_f = 0., phi_c = 0.;
+        // The final's groups: each lane's run of units, group by group, into LDS.
+        auto sums = [&](auto f32) {
+            constexpr bool F32 = decltype(f32)::value;
+            for (uint32_t g = threadIdx.x; g < sh.groups; g += blockDim.x) gs[g] = gab[g] = 0.;
+            __syncthreads();
+            uint64_t k = k0;
+            uint32_t g = k < k1 ? (uint32_t)(k / gu) : ~0u;
+            double a = 0., ab = 0.;
+            while (k < k1) {
+                const uint64_t i0 = (uint64_t)g * sh.n, ge = ((uint64_t)g + 1) * gu, ke = k1 < ge ? k1 : ge;
+                SegAcc s;
+                P::template units<F32, false>(A, (uint32_t)m, it, TAG_FINAL, k, ke, i0, i0 + sh.n, s);
+                if (F32 == MIXED) {
+                    acc.work(q, s.work);
+                    acc.st(q, 4, s.nu);
+                    acc.st(q, 5, s.nn);
+                }
+                a = s.s1;
+                ab = s.sab;
+                k = ke;
+                if (k < k1) {
+                    atomicAdd(&gs[g], a);
+                    if (F32) atomicAdd(&gab[g], ab);
+                    g++;
+                }
+            }
+            const uint32_t g0 = __builtin_amdgcn_readfirstlane(g);
+            if (__ballot(g != g0) == 0) {
+                a = wave_sum(a);
+                ab = F32 ? wave_sum(ab) : 0.;
+                if ((threadIdx.x & 63) != 0) g = ~0u;
+            }
+            if (g != ~0u) {
+                atomicAdd(&gs[g], a);
+                if (F32) atomicAdd(&gab[g], ab);
+            }
+            __syncthreads();
+            if (!first) return;
+            bool near = false;
+            double s1_big = 0., sab_big = 0., phi_small = 0.;
+            for (uint32_t i = 0; i < sh.groups; i++) {
+                const double mean = start + gs[i] / (double)sh.n;
+                if (F32) near |= fabs(mean) <= P::mixed_bound(gab[i] / (double)sh.n, start);
+                phi_small = P::phi(c, mean, coeff, phi_small);
+                s1_big += gs[i];
+                sab_big += gab[i];
+            }
+            if (F32) near |= fabs(start + s1_big / (double)sh.big) <= P::mixed_bound(sab_big / (double)sh.big, start);
+            outer_phi<P>(c, it, s1_big, phi_small, 0., 0., phi_f, phi_c);
+            redo = F32 && (near || c.redo_all) && c.phi_type == PHI_INDICATOR;
+        };
+        sums(std::integral_constant<bool, MIXED>{});
+        if (first) {
+            acc.st(q, 0, sh.big);
+            for (uint32_t i = 0; i < sh.groups; i++) acc.work(q, P::group_work(A, it));
+        }
+        if constexpr (MIXED) {
+            __syncthreads();
+            if (redo) {
+                const double f32_f = phi_f, f32_c = phi_c;
+                __syncthreads();  // redo is read before the FP64 sums write it
+                sums(std::false_type{});
+                if (first) {
+                    acc.st(q, 6, 1);
+                    acc.st(q, 7, phi_f != f32_f || phi_c != f32_c);
+                }
+            }
+        }
+        if (first) finish_outer(c, m, it, phi_f, phi_c, acc);
+        __syncthreads();  // the item and the sums are free for the next one
+    }
+    acc.template flush<true>(c);
+}
+
 // True when the fused first pass applies: both round-0 test groups (those
 // that run) fit one segment.
 template <class P>
@@ -1025,6 +1207,14 @@ hipError_t launch_batched_level(const typename P::Args& A0, uint32_t blocks, hip
     if (A.c.zero_ctl) hipLaunchKernelGGL(k_b_zero, dim3(kZeroBlocks), dim3(256), 0, s, A.c.ctl, A.c.inst_out, A.c.n_inst);
     hipError_t e = P::launch_outer(A, s);
     if (e != hipSuccess) return e;
+    if constexpr (P::kBlock) {
+        if (A.c.block) {
+            const dim3 grid((uint32_t)std::min<uint64_t>(A.c.M, kBlockGrid));
+            if (rule1) hipLaunchKernelGGL((k_b_block<P, MIXED, 1>), grid, dim3(256), 0, s, A);
+            else hipLaunchKernelGGL((k_b_block<P, MIXED, 0>), grid, dim3(256), 0, s, A);
+            return hipGetLastError();
+        }
+    }
     // Mixed form: the FP64 recheck of round r's uncertain decisions, before
     // round r + 1 reads its queue.  Its grid is the level's: a larger one
     // (measured at four times) cut the high levels' rechecked groups of

@@ -891,13 +891,46 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
         const int few = general ? 20 : fp64 ? 22 : 18, many = general ? 22 : 24;
         sh.bpc = all < (1ull << few) ? 2 : all < (1ull << many) ? 4 : 8;
     }
+    bool chosen = t != tuned.end();
     if (lanes_override) {
         sh.S = lanes_override;
+        chosen = true;
     } else if (const char* env = getenv("NMLMC_SEGMENT")) {
         const uint32_t v = (uint32_t)strtoul(env, nullptr, 10);
-        if (v) sh.S = v;
+        if (v) sh.S = v, chosen = true;
     }
+    sh.block = !chosen && block_call(M, spu, kind, form != NMLMC_FORM_MIXED, c);
     return sh;
+}
+
+// True when a level call goes to k_b_block, a block an outer sample, rather than to
+// the launch sequence: few outer samples (each takes a block's set-up and sums,
+// the sequence's launches are shared by all) whose largest count is not a long run a
+// lane (the sequence splits a long sample over the chip).  `run`: units a lane of the
+// largest count.  Measured (block against sequence, us), lines where it still wins:
+// mixed model: 1000 samples at level 3 (run 32) 78 / 134, 3000 at level 4 (64) 114 / 152,
+//   1000 at level 5 (128) 124 / 158, 300 at level 5 (128) 61 / 137; beyond: 10000 at level 3 (2) 142 /
+//   99, 2000 at level 6 (256) equal, 1000 at level 8 (1024) 1.45 times as long;
+// FP64 model: 3000 at level 2 (16) 104 / 128, 300 at level 6 (256) 76 / 107; beyond: 1000 at
+//   level 5 (128) 1.5 times as long;
+// books, mixed: 2-3 times 10^3 at level 2 (16) 0.8 of the sequence, run 64 1.2 times as long; FP64: run 16
+//   equal, 32 1.2 times as long.
+// An explicit or tuned segment, and the sequence's own settings, ask for the
+// sequence; NMLMC_BLOCK_CALLS=0/1 for either where both can take the call.
+bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) {
+    if (kind != ShapeKind::model && kind != ShapeKind::exact_book) return false;
+    if (c.ell > 0 && !c.ep.antithetic) return false;
+    if (c.cf.base % spu || c.cf.max % spu) return false;
+    if (c.ell > 0) {
+        const uint64_t most = std::max(c.cf.max, c.cc.max), least = std::min(c.cf.base, c.cc.base);
+        if (c.cc.base % spu || c.cc.max % spu || most > kRedoGroups * least) return false;
+    }
+    if (const char* e = getenv("NMLMC_BLOCK_CALLS")) return e[0] != '0';
+    if (c.redo_all || !fused_enabled() || getenv("NMLMC_FINAL_POOL") || getenv("NMLMC_TEST_SEGMENT_MIN")) return false;
+    const uint64_t run = (c.cf.max / spu + 255) / 256, base = (c.cf.base / spu + 255) / 256;
+    if (kind == ShapeKind::exact_book) return M <= 2048 && run <= (fp64 ? 8 : 16);
+    if (fp64) return (M <= 3072 && run <= 32) || (M <= 512 && run <= 256 && base <= 16);
+    return (M <= 3072 && run <= 64) || (M <= 1024 && run <= 128) || (M <= 512 && run <= 512);
 }
 
 // Times the batched level call (ell, M) of the staged problem in the current
@@ -983,10 +1016,11 @@ int Engine::sample_batched(uint32_t ell, uint64_t M, uint64_t outer_offset, uint
     // shift model, one of the reference model).
     const Shape sh = batched_shape(ell, M, mp.variant == MODEL_SHIFT ? 2 : 1, ShapeKind::model, H.c, lanes_override);
     H.c.S = sh.S;
+    H.c.block = sh.block;
     last_G = H.c.S;
     H.blocks = (uint32_t)device_cus() * sh.bpc;
     H.mixed = form == NMLMC_FORM_MIXED;
-    last_kernel = "k_b_final";
+    last_kernel = sh.block ? "k_b_block" : "k_b_final";
     return run_batched(ell, M, H.c, out, [&]() { return launch_model_batched(H, stream); }, tr_phi_f, tr_phi_c,
                        tr_nf, tr_nc);
 }

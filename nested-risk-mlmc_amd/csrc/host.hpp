@@ -137,6 +137,7 @@ struct Engine {
     // blocks of 256 threads per CU.
     struct Shape {
         uint32_t S = 0, bpc = 0;
+        uint32_t block = 0;  // 1: k_b_block instead
     };
     std::map<uint64_t, Shape> tuned;  // autotune_level's choices, key (form << 32) | level
     // Level-coupled paths for the method-2 options of portfolios staged from
@@ -147,6 +148,7 @@ struct Engine {
     // of Exact options only, another book's or a sampler class's, or those of a
     // book on level-coupled paths.
     enum class ShapeKind { model, exact_book, general, coupled };
+    static bool block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c);
     Shape batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
                         uint32_t lanes_override);
     int autotune_level(uint32_t ell, uint64_t M, Shape& best, double& best_ms);

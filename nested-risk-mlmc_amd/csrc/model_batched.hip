@@ -21,6 +21,7 @@ struct ModelPolicy {
     static constexpr uint64_t spu = (VAR == MODEL_SHIFT) ? 2 : 1;
     static constexpr bool kMulti = false;
     static constexpr bool kFuse = true;  // k_b_fused is instantiated
+    static constexpr bool kBlock = true;  // k_b_block is instantiated
     static constexpr bool kMixedWaves = true;
     static constexpr bool kTwoValued = false;
 

@@ -36,6 +36,7 @@ struct PortfolioPolicyT {
     // inner loop (BS, Exact, Unbiased) is too large to share a kernel with the
     // outer draw and the final at a useful occupancy.
     static constexpr bool kFuse = EXACT_ONLY;
+    static constexpr bool kBlock = EXACT_ONLY && !MULTI;
     // The general inner loop (FP64 Unbiased paths beside the FP32 Exact terms)
     // runs without the mixed form's register cap.
     static constexpr bool kMixedWaves = EXACT_ONLY;

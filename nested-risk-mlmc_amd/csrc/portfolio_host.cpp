@@ -351,6 +351,7 @@ int Engine::sample_portfolio_batched(uint32_t ell, uint64_t M, uint64_t outer_of
                                         : ShapeKind::general;
     const Shape sh = batched_shape(ell, M, 1, kind, H.c, lanes_override);
     H.c.S = sh.S;
+    H.c.block = sh.block;
     last_G = H.c.S;
     if ((rc = ensure_pf_R(std::min(M, batched_chunk())))) return rc;
     H.R_tau = pf_R;
@@ -359,7 +360,7 @@ int Engine::sample_portfolio_batched(uint32_t ell, uint64_t M, uint64_t outer_of
     H.mixed = form == NMLMC_FORM_MIXED;
     H.multi = false;
     H.R32 = (H.mixed && H.exact_only) ? pf_R32 : nullptr;
-    last_kernel = "k_b_final";
+    last_kernel = sh.block ? "k_b_block" : "k_b_final";
     return run_batched(ell, M, H.c, out, [&]() { return launch_portfolio_batched(H, stream); }, tr_phi_f,
                        tr_phi_c, tr_nf, tr_nc);
 }

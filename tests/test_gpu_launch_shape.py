@@ -14,6 +14,7 @@ SCAL = dict(r=0.05, rho=0.2, tau=0.02, dt_h0inv=8, dt_beta=4, dt_prob_expo=-1.5,
 
 
 def _check(nm, monkeypatch, ell, M, segment):
+    monkeypatch.setenv("NMLMC_BLOCK_CALLS", "0")
     got = nm.sample(ell, M, outer_offset=0, trace=True)
     assert nm.last_group_lanes() == segment, (ell, M, nm.last_group_lanes())
     monkeypatch.setenv("NMLMC_SEGMENT", "7")
