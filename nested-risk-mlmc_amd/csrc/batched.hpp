@@ -37,7 +37,7 @@ constexpr int kMaxClasses = 32;
 // Relative bound (times the mean magnitude of the inner terms) on the FP32
 // inner mean's error.  FP32 normals lie within about 2^-20 of the FP64 ones
 // (boxmuller_f32 takes the radius of the words whose float rounds to 1 from
-// the complement word) and the compensated sums add 2^-23.
+// the complement word); the terms are added in FP64.
 constexpr double kMixedBound = 0x1p-16;
 // FP64 redo of the mixed form: the first kRedoSlots listed outer samples with at
 // most kRedoGroups final groups are split over up to kRedoParts blocks each

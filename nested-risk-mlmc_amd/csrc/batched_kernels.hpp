@@ -2,7 +2,8 @@
 // policy P and on the precision of the inner arithmetic.
 //
 // Launch order of one level call (launch_batched_level):
-//   [k_b_zero unless the control block is clear already], [P's outer-draw kernel], k_b_init and k_b_test(r) for r = 0..R-1
+//   [k_b_zero unless the control block is clear already], [P's outer-draw kernel], then
+//   k_b_block alone (small calls), or k_b_init and k_b_test(r) for r = 0..R-1
 //   (or k_b_fused and k_b_test(r) for r = 1..R-1), k_b_final_count (its
 //   last block lays the final pool out), k_b_final_fill, k_b_final, [k_b_redo_split and
 //   k_b_redo_seq when MIXED]
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(256) void k_b_init(typename P::Args A) {
 // Mixed form: true when the refinement decision taken from FP32-accumulated
 // sums may differ from the one the FP64 sums of the same draws give (the
 // batched FP64 form's).  With |s1 - s1_64| <= e1 and |s2 - s2_64| <= e2
-// (P::decision_bounds, plus 2^-21 s2 for the compensated sums' own rounding),
+// (P::decision_bounds, plus 2^-21 s2 for the sums' own rounding),
 // |dist - dist_64| <= ed = e1 / n and |var - var_64| <= ev (both a sixteenth larger,
 // which leaves room for the FP64 sums' own rounding, at most n 2^-53 of the terms'
 // magnitudes: a sixteenth of e1 at n = 2^30), so delta^2_64 lies in
