@@ -860,6 +860,10 @@ uint64_t Engine::batched_chunk() {
 // about 4 us a launch), and the FP64 kernels hold two or three a CU at a time: 2 a
 // CU for few units (a call of 1000 mixed samples 174 -> 128 us), 4 up to 2^24, then
 // 8, which balance better (10^7 samples of the model, not adaptive: 1015 -> 915 us).
+//
+// Calls whose differences may be rounding residues (residue_call) keep the segment
+// that fixes those residues: the largest of 64, 32, 16 or 8 units that leaves 2^19
+// segments, else 16, or 4 from 1024 units on.
 Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
                                     uint32_t lanes_override) {
     if (force.S) return force;
@@ -868,6 +872,7 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
     if (t != tuned.end()) {
         sh = t->second;
     } else {
+        const bool residues = residue_call(M, kind, form != NMLMC_FORM_MIXED, c);
         const bool adaptive = c.cf.max > 2 * c.cf.base, fp64 = form != NMLMC_FORM_MIXED;
         const uint64_t group = adaptive ? c.cf.base : c.cf.max;
         const uint64_t units = (group + spu - 1) / spu;
@@ -887,6 +892,11 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
             if (whole) sh.S = std::max(sh.S, pow2_ceil_u32(units));
         }
         if (kind == ShapeKind::coupled && all < (1ull << 18)) sh.S = std::min(sh.S, 2u);
+        if (residues) {
+            sh.S = units >= 1024 ? 4 : 16;
+            for (uint32_t S : {8u, 16u, 32u, 64u})
+                if (m * ((units + S - 1) / S) >= (1ull << 19)) sh.S = std::max(sh.S, S);
+        }
         const bool general = kind == ShapeKind::general || kind == ShapeKind::coupled;
         const int few = general ? 20 : fp64 ? 22 : 18, many = general ? 22 : 24;
         sh.bpc = all < (1ull << few) ? 2 : all < (1ull << many) ? 4 : 8;
@@ -901,6 +911,22 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
     }
     sh.block = !chosen && block_call(M, spu, kind, form != NMLMC_FORM_MIXED, c);
     return sh;
+}
+
+// True for the FP64 model's antithetic levels with a loss that is no indicator and
+// fewer than 2^15 outer samples.  There phi_fine - phi_coarse of an outer sample whose
+// groups all lie on one side of the threshold is 0 but for the last places of its
+// means, and a call may hold no other kind (at level 8 some 250 outer samples, a
+// dozen above the threshold): its difference sums are then residues of the order in
+// which the inner samples were added, 10^-16 and of either sign.  The order is part
+// of such a call's results, so it does not follow the tuning of other calls: own
+// segments (batched_shape), the launch sequence and its Box-Muller pair
+// (boxmuller_f64_lib).  The non-adaptive sweep pays 110 us at its levels 6 to 8 (1954, 691 and
+// 245 outer samples), which k_b_block would take: 1180 us instead of 1070.
+// From 2^15 samples on, hundreds straddle the threshold at the levels that have so
+// many (2^15 at level 3: some 80), and their differences exceed residues 10^12 times.
+bool Engine::residue_call(uint64_t M, ShapeKind kind, bool fp64, const BatchedCommon& c) {
+    return kind == ShapeKind::model && fp64 && c.ell > 0 && c.ep.antithetic && c.phi_type != PHI_INDICATOR && M < (1ull << 15);
 }
 
 // True when a level call goes to k_b_block, a block an outer sample, rather than to
@@ -927,6 +953,7 @@ bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, con
     }
     if (const char* e = getenv("NMLMC_BLOCK_CALLS")) return e[0] != '0';
     if (c.redo_all || !fused_enabled() || getenv("NMLMC_FINAL_POOL") || getenv("NMLMC_TEST_SEGMENT_MIN")) return false;
+    if (residue_call(M, kind, fp64, c)) return false;
     const uint64_t run = (c.cf.max / spu + 255) / 256, base = (c.cf.base / spu + 255) / 256;
     if (kind == ShapeKind::exact_book) return M <= 2048 && run <= (fp64 ? 8 : 16);
     if (fp64) return (M <= 3072 && run <= 32) || (M <= 512 && run <= 256 && base <= 16);
