@@ -37,7 +37,10 @@ int set_error(int code, const char* fmt, ...) {
     return code;
 }
 
+// The thread's last error is cleared with the report: the launches' checks read it,
+// and one left standing would make a launch that ran look failed.
 int hip_fail(hipError_t e, const char* what) {
+    (void)hipGetLastError();
     return set_error(NMLMC_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
@@ -119,8 +122,7 @@ void Engine::free_samplers() {
     if (d_states) hipFree(d_states);
     if (d_partials) hipFree(d_partials);
     if (d_ws) hipFree(d_ws);
-    if (d_help) hipFree(d_help);
-    d_help = nullptr;
+    drop_help();
     d_states = nullptr;
     d_partials = nullptr;
     d_ws = nullptr;
@@ -184,6 +186,18 @@ PlainHelp* Engine::ensure_help() {
     }
     help_base = 0;
     return d_help;
+}
+
+// Gives the postings up once no kernel uses them: the next call starts from cleared
+// counters.  After any failure of a call that may have run, when what the device
+// counted is not known.
+void Engine::drop_help() {
+    if (!d_help) return;
+    if (stream) hipStreamSynchronize(stream);
+    hipFree(d_help);
+    (void)hipGetLastError();
+    d_help = nullptr;
+    help_base = 0;
 }
 
 int Engine::ensure_ws(size_t n) {
@@ -390,15 +404,23 @@ int Engine::sample_model_parity(uint32_t ell, uint64_t M, uint32_t lanes_overrid
     H.tr_nc = tb.nc;
     hipError_t e = hipEventRecord(ev0, stream);
     if (e != hipSuccess) return hip_fail(e, "hipEventRecord");
+    auto failed = [&](hipError_t err, const char* what) {
+        if (H.help) drop_help();
+        return hip_fail(err, what);
+    };
+    (void)hipGetLastError();  // other code's, if any: not this launch's
     e = launch_model_parity(H, stream);
-    if (e != hipSuccess) return hip_fail(e, "launch k_model_parity");
+    if (e != hipSuccess) return failed(e, "launch k_model_parity");
     if (H.help) help_base += H.blocks;
-    if ((e = hipEventRecord(ev1, stream)) != hipSuccess) return hip_fail(e, "hipEventRecord");
+    if ((e = hipEventRecord(ev1, stream)) != hipSuccess) return failed(e, "hipEventRecord");
     e = launch_reduce_partials(parts, (uint32_t)nblocks, res, stream);
-    if (e != hipSuccess) return hip_fail(e, "launch k_reduce_partials");
+    if (e != hipSuccess) return failed(e, "launch k_reduce_partials");
     last_kernel = "k_model_parity";
     rc = finish_call(ell, out, res);
-    if (rc) return rc;
+    if (rc) {
+        if (H.help) drop_help();
+        return rc;
+    }
     rc = trace_finish(M, tb, tr_phi_f, tr_phi_c, tr_nf, tr_nc);
     if (rc) return rc;
     return set_error(NMLMC_OK, "");

@@ -65,6 +65,7 @@ struct Engine {
     PlainHelp* d_help = nullptr;      // postings of the plain model calls
     uint32_t help_base = 0;           // its counters: blocks of the calls so far
     PlainHelp* ensure_help();
+    void drop_help();
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // Scratch of a plain-form level call: the per-block partial records (room

@@ -13,6 +13,7 @@
 // equal those of the sequential reference.
 #include "engine.hpp"
 #include "model.hpp"
+#include "plain_help.hpp"
 
 namespace nmlmc {
 
@@ -208,7 +209,7 @@ __device__ __forceinline__ void help_others(const ModelParams& mp, PlainHelp* h,
                 if (seg < 0) slot = -1;
             }
             if (lane == 0) {
-                if (slot < 0 && (shared_load(&h->ended) - base == gridDim.x || shared_load(&h->started) - base < gridDim.x))
+                if (slot < 0 && helper_leaves(shared_load(&h->started), shared_load(&h->ended), base, gridDim.x))
                     slot = -2;
                 job[0] = slot;
                 job[1] = seg;
