@@ -42,10 +42,12 @@ struct ModelPolicy {
     // Mixed form, refinement decisions: bounds on |s1 - s1_64| and |s2 - s2_64|
     // of n FP32 terms (their error scales sum to sab, squared to smm) against
     // the FP64 sums of the same draws.  Each FP32 term is within
-    // e_i = 2^-19 (mag_i + 1) of its FP64 value (normals within 2^-20.5, float
-    // rounding of Y and of the products 2^-23 of mag), so |s1 - s1_64| is at
-    // most 2^-19 (sab + n) and |s2 - s2_64| <= sum(2 |d_i| e_i + e_i^2) with
-    // |d_i| <= mag_i.
+    // e_i = 2^-19 (mag_i + 1) of its FP64 value: the normals are off by at most
+    // 2^-19.93 (1 + |z|) (bm_polar_f32), float rounding of Y and of the products adds
+    // 2^-23 mag; a term p^2 - q^2 of the reference model, mag = p^2 + q^2, by
+    // 2 |p| dp + 2 |q| dq <= (mag + 1) (dp^2 + dq^2)^(1/2) and dp, dq below 2^-19.5 where mag is not
+    // itself some 10.  So |s1 - s1_64| is at most 2^-19 (sab + n) and
+    // |s2 - s2_64| <= sum(2 |d_i| e_i + e_i^2) with |d_i| <= mag_i.
     __device__ static void decision_bounds(double n, double, double sab, double smm, double& e1, double& e2) {
         e1 = 0x1p-19 * (sab + n);
         e2 = 0x1p-17 * (smm + sab) + 0x1p-36 * n;

@@ -85,7 +85,8 @@ __device__ __forceinline__ double inner_bs_d(const PortfolioDevice& pf, const Op
     return val + cv;
 }
 
-// e^x: x = k ln 2 + (f + fl), |f| <= ln(2) / 2, and a minimax polynomial for e^f
+// e^x: x = k ln 2 + (f + fl), |f| <= ln(2) / 2 (Cody and Waite's reduction with its remainder
+// kept), and a minimax polynomial for e^f
 // (error below 2^-57); 1 + f is summed with its rounding error, so the result is the
 // nearest double but for a few in a hundred.  Straight-line code for |x| below 2^29
 // (beyond the range of a double, infinity or 0); the arguments here are log returns.

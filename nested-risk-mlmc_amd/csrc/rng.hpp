@@ -81,8 +81,10 @@ __device__ __forceinline__ double i64_to_f64(uint64_t u) {
 }
 
 // The three functions of the FP64 Box-Muller pair on just the arguments it
-// meets, in straight-line code.  Their polynomials are minimax fits computed
-// for these ranges; the errors left are below 2^-57.
+// meets, in straight-line code.  The reductions are the classical ones (fdlibm's log by
+// s = f / (2 + f) and its cosine with the rounding of 1 - t / 2 carried, Cody and Waite's
+// two-part constants); the polynomials are minimax fits computed for these ranges, which
+// leave less than 2^-57.
 //
 // log u, u in (0, 1]: u = 2^e m with m in [sqrt(1/2), sqrt 2), f = m - 1,
 // s = f / (2 + f), and log m = 2 atanh s = f - s (f - R) with R = s^2 (2/3 +
@@ -186,23 +188,28 @@ __device__ __forceinline__ void boxmuller_f64_lib(uint64_t u0, uint64_t u1, doub
 // u0 -> [-1,1], sin/cos(pi x) and log by the hardware's instructions, as the
 // polar parts of the pair (r sn, r cs) and r2 = r^2.
 //
-// The angle goes in revolutions, which is what the instructions take: u0 2^-65
-// from its high word, off by at most 2^-33 (an angle error below 2^-30).  The
-// float of u1 carries a relative error of about 2^-24, i.e. an absolute error
-// of that in ln u1; the radius r = sqrt(-2 ln u1) then has an error of
-// about 2^-24 / r, which for u1 near 1 (small r) would reach 100% (a word of
-// u1 >= 2^64 - 2^39 rounds to 1: radius 0 against an FP64 radius up to 2^-12).
-// Words with u1 > 1 - 2^-8 (top byte all ones, 2^-8 of them) therefore take
-// the radius from q = 1 - u01(u1) = ~u1 2^-64 + 2^-65, whose float is accurate
-// to 2^-24 relative: -ln(1 - q) = q (1 + q/2 + q^2/3 + q^3/4), truncation below
-// 2^-33 relative for q <= 2^-8.  Elsewhere r >= 2^-3.5 and the normals stay
-// within 2^-20.5 (2^-19 for u1 below 2^-20, which 2^-20 of the words have).
+// The angle goes in revolutions, which is what the instructions take: u0 2^-64 from
+// its high word, off by at most 2^-32 for the low word and 2^-26 for the rounding of
+// the high word to a float, 2^-23.3 of an angle.  The float of u1 carries a relative
+// error of about 2^-24, i.e. an absolute error of that in ln u1; the radius
+// r = sqrt(-2 ln u1) then has an error of about 2^-24 / r, which for u1 near 1
+// (small r) would reach 100% (a word of u1 >= 2^64 - 2^39 rounds to 1: radius 0
+// against an FP64 radius up to 2^-12).  Words with u1 > 1 - 2^-8 (top byte all ones,
+// 2^-8 of them) therefore take the radius from q = 1 - u01(u1) = ~u1 2^-64 + 2^-65,
+// whose float is accurate to 2^-24 relative: -ln(1 - q) = q (1 + q/2 + q^2/3 + q^3/4),
+// truncation below 2^-33 relative for q <= 2^-8.
+//
+// Error of a normal z = r sn or r cs: at most 2^-19.93 (1 + |z|), from all 2^32 high
+// words of either argument (low words 0, 2^31 and 2^32 - 1): sine and cosine off by at
+// most 2^-22.33 (2^-23.32 where below 2^-10), the radius by 2^-21.4 below 0.1,
+// 2^-22 up to 2, 2^-21 up to 4, and at the largest (2^-32 of the words) 2^-20.3.  rms over random
+// words 2^-23.3.
 //
 // Bound by VALU issue, as the Threefry block before it.  Whole-word conversions
 // (a shift, clamp and scaling each), the C functions' denormal steps and the
 // correctly rounded root took 85 slots of 64 lanes after a block of 116; this
-// way 11, with an error no larger anywhere in 2^20 pairs (edges included): at
-// most 2^-20.5 against 2^-19.8, rms 2^-23.3 against 2^-22.9.
+// way 11, with an error no larger: over 2^20 pairs, edges included, at most 2^-20.5
+// against 2^-19.8, rms 2^-23.3 against 2^-22.9.
 __device__ __forceinline__ void bm_polar_f32(uint64_t u0, uint64_t u1, float& sn, float& cs, float& r, float& r2) {
     const float h = (float)(int32_t)(u0 >> 32) * 0x1p-32f;
     sn = __builtin_amdgcn_sinf(h);
