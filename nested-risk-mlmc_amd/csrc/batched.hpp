@@ -35,9 +35,12 @@ constexpr int kMaxRounds = 30;
 constexpr int kMaxClasses = 32;
 
 // Relative bound (times the mean magnitude of the inner terms) on the FP32
-// inner mean's error.  FP32 normals lie within about 2^-20 of the FP64 ones
-// (boxmuller_f32 takes the radius of the words whose float rounds to 1 from
-// the complement word); the terms are added in FP64.
+// inner mean's error.  FP32 normals lie within 2^-19.93 (1 + |z|) of the FP64 ones
+// (bm_polar_f32, which takes the radius of the words whose float rounds to 1 from
+// the complement word).  The terms and their error scales are added in FP64 (the
+// model, books of Exact options) or in compensated FP32 (the FP32 Exact terms of other
+// books); books' second-moment scales, sums of positive terms over a lane's run, in
+// plain FP32.
 constexpr double kMixedBound = 0x1p-16;
 // FP64 redo of the mixed form: the first kRedoSlots listed outer samples with at
 // most kRedoGroups final groups are split over up to kRedoParts blocks each

@@ -129,17 +129,16 @@ struct ModelPolicy {
             return;
         }
         if (VAR == MODEL_SHIFT && ((i0 | i1) & 1) == 0) {
-            double az = 0., aq = 0.;
-            float br = 0.f;
+            double az = 0., aq = 0., br = 0.;
             for (uint64_t u = u0; u < u1; u++) {
                 const u64x2 w = threefry2x64_20(0, base | u, A.c.seed, k1);
                 float sn, cs, r, r2;
                 bm_polar_f32(w.a, w.b, sn, cs, r, r2);
                 az += (double)((sn + cs) * r);
-                br += r;
+                br += (double)r;
                 if (TEST) aq += (double)r2;
             }
-            const double n = (double)cnt, aY = fabs(Y), ar = 0x1.6a09e667f3bcdp+0 * (double)br;
+            const double n = (double)cnt, aY = fabs(Y), ar = 0x1.6a09e667f3bcdp+0 * br;
             s.s1 += n * Y + az;
             s.sab += n * aY + ar;
             if (TEST) {

@@ -176,3 +176,19 @@ def test_mixed_sums_within_the_decision_bounds(probe, variant, tau, count):
     assert np.all(np.abs(s1 - d[0]) <= 2.0 ** -19 * (sab + count))
     assert np.all(np.abs(s2 - d[1]) <= 2.0 ** -17 * (smm + sab) + 2.0 ** -36 * count)
     assert np.all(sab * (1 + 2.0 ** -20) >= np.abs(d[0])) and np.all(smm * (1 + 2.0 ** -20) >= d[1])
+
+
+def test_error_scale_of_a_long_run(probe):
+    """The scale of 2^17 pairs in one lane is that of the same pairs in 2^11 lanes: sums of
+    positive FP64 terms, at most 2^17 2^-53 apart."""
+    pairs, parts = 1 << 17, 1 << 11
+    one = probe[1](1, True, 0.5, 3, 2 * pairs, [0.25], [9], [0], [pairs])
+    u = np.arange(parts) * (pairs // parts)
+    many = probe[1](1, True, 0.5, 3, 2 * pairs, np.full(parts, 0.25), np.full(parts, 9), u, u + pairs // parts)
+    for k in (2, 3):
+        assert abs(one[k][0] / many[k].sum() - 1) <= pairs * U
+    # And it is sqrt(2) times the radii's sum, to the FP32 radii's error.
+    b = np.arange(pairs, dtype=np.uint64)
+    w = threefry2x64_20(0, (np.uint64(65) << np.uint64(40)) | b, 3, 9)
+    r = np.sqrt(-2 * np.log(w[1].astype(np.float64) * 2.0 ** -64 + 2.0 ** -65))
+    assert abs(one[2][0] / (2 * pairs * 0.25 + np.sqrt(2) * r.sum()) - 1) <= 2.0 ** -20
