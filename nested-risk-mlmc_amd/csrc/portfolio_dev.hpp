@@ -86,8 +86,7 @@ __device__ __forceinline__ double inner_bs_d(const PortfolioDevice& pf, const Op
 }
 
 // e^x: x = k ln 2 + (f + fl), |f| <= ln(2) / 2 (Cody and Waite's reduction with its remainder
-// kept), and a minimax polynomial for e^f
-// (error below 2^-57); 1 + f is summed with its rounding error, so the result is the
+// kept), and a minimax polynomial for e^f (error below 2^-57); 1 + f is summed with its rounding error, so the result is the
 // nearest double but for a few in a hundred.  Straight-line code for |x| below 2^29
 // (beyond the range of a double, infinity or 0); the arguments here are log returns.
 __device__ __forceinline__ double exp_d(double x) {
@@ -576,14 +575,18 @@ __device__ __forceinline__ float inner_exact_f(const PortfolioDevice& pf, const 
 }
 
 // inner_exact_f from an option's MixRec: the term already divided by p and its
-// error scale `mag`, such that 2^-18 mag bounds (with a factor 4 to spare) the
-// difference between this FP32 term and the FP64 term of the same draws.  R: the
-// stock's level at tau over S0.
+// error scale `mag`, such that 2^-18 mag bounds the difference between this FP32 term
+// and the FP64 term of the same draws.  R: the stock's level at tau over S0.
 //
-// The levels S carry a relative error of about 2^-20.5 at most (the FP32 normals'
-// error times sigma sqrt(T), plus a few units of 2^-24 from the exponentials of
-// O(1) arguments), and so their continuous functions, the payoffs and (R - 1) S of
-// the control variate, an error of about 2^-20 (S1 + S2 + S_t) (1 + |R - 1|) |hdiscp|.
+// The levels S carry a relative error eps: sigma sqrt(T) times the FP32 normals'
+// 2^-19.93 (1 + |z|), which is below 2^-19.2 but for 10^-7 of the pairs (radius above 5.7)
+// and 2^-18.4 at the end of their range, and some 2^-21 from the arguments and results of the
+// exponentials.  Their continuous functions, the payoffs and (R - 1) S of the control
+// variate, are then within eps (S1 + S2 + 2 S_t + |R - 1| (S1 + S2)) |hdiscp| <= eps mag: inside
+// 2^-18 mag for every draw up to sigma sqrt(T) = 1, and for a group's sum far beyond that
+// (rms of eps 2^-23.3 sigma sqrt(T)).  What does not shrink with the levels has a term of its
+// own, 2^-5 (K + 1): payoffs of a put round at 2^-24 K however small S is (four of them in
+// v: 2^-22 K |hdiscp| at most), and a digital's coefficient at 2^-24 |hdiscp|.
 // A digital payoff, or the control variate's indicator [S < K], whose stock level
 // lies within 2^-17 K of the strike may jump under that rounding; the jump's size
 // enters mag with the weight 2^18, so that the bound covers it whole.
@@ -592,7 +595,7 @@ __device__ __forceinline__ float inner_exact_f(const PortfolioDevice& pf, const 
 // sample, and by the gathers (guide, record, stock, level).  The payoff of either
 // kind is one median: d = m sgn (S - K) clamped to [0, cap], with m = 1 and no cap
 // for a vanilla, m = 2^60 and cap 1 for a digital.  With levels in units of S0 (four
-// constants a stock), sums in FP64, an error scale of five instructions and a search
+// constants a stock), sums in FP64, an error scale of six instructions and a search
 // without the checks of its bounds, the large book's sweep took 9.2 ms before and 8.06
 // after, 16 books with their staging 13.1 and 11.5 ms.
 __device__ __forceinline__ float inner_exact_mix(const MixRec& q, const MixStock& st, bool anti, bool cv_on,
@@ -614,7 +617,7 @@ __device__ __forceinline__ float inner_exact_mix(const MixRec& q, const MixStock
     const float itm = (d1 > 0.f ? S1 : 0.f) + (d2 > 0.f ? S2 : 0.f);
     const float v = __builtin_fmaf(cvf, itm, __builtin_fmaf(-2.f, pt, p1 + p2));
     const float h = fabsf(q.hdiscp);
-    mag = (2.f * h) * ((S1 + S2 + St) * (1.f + fabsf(cvf)));
+    mag = (2.f * h) * __builtin_fmaf(S1 + S2 + St, 1.f + fabsf(cvf), __builtin_fmaf(q.K, 0x1p-5f, 0x1p-5f));
     const float win = 0x1p-17f * fabsf(Km);
     if (fminf(fminf(fabsf(d1), fabsf(d2)), fabsf(dt)) < win) {  // some 10^-5 of the samples
         const float n12 = (float)(fabsf(d1) < win) + (float)(fabsf(d2) < win);

@@ -15,7 +15,8 @@ Bounds, in units of 2^-53 of the value unless said otherwise:
   2^-10), the radius by 2^-20.3, and together 2^-19.93 (1 + |z|);
 - mixed sums of a draw group: the refinement's bounds e1 = 2^-19 (sab + n) and
   e2 = 2^-17 (smm + sab) + 2^-36 n, which the FP32 pairs' error above and the FP32 operations
-  (2^-23 of mag) leave room for."""
+  (2^-23 of mag) leave room for;
+- the mixed Exact term: 2^-18 of its error scale, for every draw up to sigma sqrt(T) = 1."""
 import ctypes as C
 import os
 
@@ -176,6 +177,30 @@ def test_mixed_sums_within_the_decision_bounds(probe, variant, tau, count):
     assert np.all(np.abs(s1 - d[0]) <= 2.0 ** -19 * (sab + count))
     assert np.all(np.abs(s2 - d[1]) <= 2.0 ** -17 * (smm + sab) + 2.0 ** -36 * count)
     assert np.all(sab * (1 + 2.0 ** -20) >= np.abs(d[0])) and np.all(smm * (1 + 2.0 ** -20) >= d[1])
+
+
+@pytest.mark.parametrize("anti", [True, False])
+@pytest.mark.parametrize("cv", [True, False])
+@pytest.mark.parametrize("tau", [1.0 / 52, 0.2])
+def test_mixed_exact_term_within_its_scale(probe, anti, cv, tau):
+    """Vanillas and digitals near and far from the money, strikes within 2^-17 of the level
+    among them (the FP64 level of the draw itself, and both sides of the window)."""
+    u0, u1 = _pairs()
+    n = len(u0)
+    rs = np.random.RandomState(17)
+    S0, T = 10.0 ** rs.uniform(-3, 5, n), rs.uniform(0.25, 4, n)
+    sigma = rs.uniform(0.05, 1, n) / np.sqrt(T)
+    R = np.exp(rs.normal(0, 0.3, n)).astype(np.float32).astype(np.float64)
+    typ = rs.choice([1., -1., 2., -2.], n)
+    x, y, _ = (v.astype(np.float64) for v in _reference(u0, u1))
+    drift = 0.05 - sigma * sigma / 2
+    g = np.exp(sigma * np.sqrt(T - tau) * y + drift * (T - tau))
+    levels = [R * S0 * g] + [S0 * np.exp(s * sigma * np.sqrt(tau) * x + drift * tau) * g for s in (1, -1)]
+    at = np.choose(rs.randint(0, 3, n), levels) * (1 + rs.choice([0, 1, -1], n) * 2.0 ** rs.uniform(-24, -15, n))
+    K = np.where(rs.uniform(size=n) < 0.3, at, S0 * np.exp(rs.normal(0, 0.3, n)))
+    K = np.clip(K, 1e-6 * S0, 1e6 * S0)
+    f, mag, d = probe[2](0.05, tau, anti, cv, np.array([S0, sigma, K, T, rs.standard_t(3, n), R, typ]), np.array([u0, u1]))
+    assert np.all(np.isfinite(f)) and np.all(np.abs(f - d) <= 2.0 ** -18 * mag)
 
 
 def test_error_scale_of_a_long_run(probe):
