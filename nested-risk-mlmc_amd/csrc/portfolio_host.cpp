@@ -221,19 +221,28 @@ int Engine::stage_portfolio(const portfolio_data* data) {
     if (P.coupled && data->subsample != 1)
         return set_error(NMLMC_ERR_ARG, "level-coupled paths need sub-sampling mode 1");
     // The book is valid: its tables replace the staged ones.  The block is used again
-    // when it fits (work on the tables is ordered on the engine's stream).
+    // when it fits (work on the tables is ordered on the engine's stream).  From here on
+    // the earlier book's tables are gone: if a step fails, no book is staged, and
+    // nothing is left in flight from the pinned memory.
+    if (problem == PROBLEM_PORTFOLIO) problem = -1;
+    std::memset(&pf, 0, sizeof(pf));
     for (void* p : pf_allocs) hipFree(p);
     pf_allocs.clear();
+    auto failed = [this](hipError_t err, const char* what) {
+        hipStreamSynchronize(stream);
+        return hip_fail(err, what);
+    };
     hipError_t e;
     if (size > pf_blob_cap || pf_blob_cap > 4 * size + ((size_t)1 << 20)) {
         free_portfolio();
-        problem = -1;  // nothing is staged if the allocation fails
         if ((e = hipMalloc(&pf_blob, size)) != hipSuccess) return hip_fail(e, "hipMalloc portfolio tables");
         pf_blob_cap = size;
     }
     char* const dev = (char*)pf_blob;
     if ((e = hipMemcpyAsync(dev, host, up, hipMemcpyHostToDevice, stream)) != hipSuccess)
-        return hip_fail(e, "hipMemcpy portfolio tables");
+        return failed(e, "hipMemcpy portfolio tables");
+    // Test hook: NMLMC_TEST_STAGE_FAIL=1 fails here, the tables half replaced.
+    if (getenv("NMLMC_TEST_STAGE_FAIL")) return failed(hipErrorUnknown, "portfolio tables (test hook)");
     StageArgs S{};
     for (int m = 0; m < 3; m++) {
         P.options[m] = (const OptionRec*)(dev + o_opt[m]);
@@ -257,8 +266,8 @@ int Engine::stage_portfolio(const portfolio_data* data) {
     S.prob_norm = P.prob_norm;
     S.subsample = P.subsample;
     S.options_count = P.options_count;
-    if ((e = launch_stage(S, stream)) != hipSuccess) return hip_fail(e, "launch k_stage");
-    if ((e = hipEventRecord(stage_ev, stream)) != hipSuccess) return hip_fail(e, "hipEventRecord staging");
+    if ((e = launch_stage(S, stream)) != hipSuccess) return failed(e, "launch k_stage");
+    if ((e = hipEventRecord(stage_ev, stream)) != hipSuccess) return failed(e, "hipEventRecord staging");
     if (h_stage_cap > kStageKeep) free_stage();
     // Work of one init_inner_sampler call without sub-sampling: the BS options.
     pf_bs_work = 0.;
