@@ -43,9 +43,9 @@ struct PortfolioParityArgs {
     uint64_t* tr_nc;
 };
 
-// Waves a virtual thread may take, and the doubles of LDS scratch a block
-// needs beyond R_tau and z: the wave sums of a block of up to kMaxW waves (3
-// each), or thread 0's broadcast (11 values).
+// Waves a virtual thread may take, and the doubles of LDS scratch an inner loop
+// needs: the wave sums of a block of up to kMaxW waves (3 each), or thread 0's
+// broadcast (11 values).
 constexpr uint32_t kMaxW = 8;
 constexpr uint32_t kParityRed = 32;
 static_assert(3 * kMaxW <= kParityRed && 11 <= kParityRed, "LDS reduction scratch");
@@ -357,10 +357,11 @@ __device__ __forceinline__ InnerSums general_inner(const PortfolioParityArgs& A,
 
 // inner_sampler::sample_inner (nested_sampler.hpp:131-161) over `count` samples
 // from the thread's streams (ss: sync, si: inner), block-uniform result.  red:
-// LDS scratch of at least 3 W doubles.
+// LDS scratch of kParityRed doubles; sc: the general kernel's.
 template <uint32_t W, int KIND>
 __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, const double* R, uint64_t k1,
-                                                  StreamState& ss, StreamState& si, uint64_t count, double* red) {
+                                                  StreamState& ss, StreamState& si, uint64_t count, double* red,
+                                                  GeneralScratch* sc) {
     constexpr bool EXACT_ONLY = KIND == PAR_EXACT;
     const PortfolioDevice& pf = A.pf;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -456,8 +457,7 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
     }
     if constexpr (KIND == PAR_GENERAL) {
         static_assert(W == 1, "one wave a virtual thread");
-        __shared__ GeneralScratch sc;
-        if (pf.subsample != 0) return general_inner(A, R, k1, ss, si, count, sc);
+        if (pf.subsample != 0) return general_inner(A, R, k1, ss, si, count, *sc);
     }
     // Reference loop on thread 0.
     if (tid == 0) {
@@ -544,23 +544,32 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
 #define NMLMC_PLAIN_GENERAL_WAVES 2
 #endif
 
+// Doubles of LDS that the outer draw's normals and the inner loops' scratch take by turns.
+__host__ __device__ constexpr uint32_t lds_shared_doubles(bool general, uint32_t d) {
+    const uint32_t scratch = kParityRed + (general ? (uint32_t)(sizeof(GeneralScratch) / sizeof(double)) : 0u);
+    return d > scratch ? d : scratch;
+}
+static_assert(sizeof(GeneralScratch) % sizeof(double) == 0, "LDS layout in doubles");
+
 template <uint32_t W, int KIND>
 __global__ __launch_bounds__(64 * W, (KIND == PAR_EXACT ? NMLMC_PLAIN_EXACT_WAVES : KIND == PAR_NO_UNBIASED ? NMLMC_PLAIN_NO_UNBIASED_WAVES : NMLMC_PLAIN_GENERAL_WAVES)) void k_portfolio_parity(
     PortfolioParityArgs A) {
     constexpr bool EXACT_ONLY = KIND == PAR_EXACT;
-    // R_tau[d], z[d], reduction scratch[kParityRed], then the moment sums, which
-    // thread 0 keeps (in registers, 32 doubles in every lane, they spilled).
+    // The moment sums, which thread 0 keeps (in registers, 32 doubles in every lane,
+    // they spilled); the inner loops' scratch, and in its place z[d], the outer draw's
+    // normals; R_tau[d].
     extern __shared__ double smem[];
     const PortfolioDevice& pf = A.pf;
     const EngineParams& ep = A.ep;
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     const uint64_t k1 = t;
     const uint32_t d = pf.d;
-    double* R = smem;
-    double* z = smem + d;
-    double* red = smem + 2 * d;
-    double* f_sums = red + kParityRed;
+    double* f_sums = smem;
     double* d_sums = f_sums + kMaxPhi * kMaxMoments;
+    double* z = d_sums + kMaxPhi * kMaxMoments;
+    double* red = z;
+    GeneralScratch* sc = KIND == PAR_GENERAL ? reinterpret_cast<GeneralScratch*>(red + kParityRed) : nullptr;
+    double* R = z + lds_shared_doubles(KIND == PAR_GENERAL, d);
     if (tid == 0)
         for (int i = 0; i < kMaxPhi * kMaxMoments; i++) f_sums[i] = d_sums[i] = 0.;
 
@@ -643,7 +652,7 @@ __global__ __launch_bounds__(64 * W, (KIND == PAR_EXACT ? NMLMC_PLAIN_EXACT_WAVE
                 n = (fine_only || ep.antithetic) ? small : group == 0 ? nf : nc;
             }
             if (!decided) {
-                const InnerSums s = parity_inner<W, KIND>(A, R, k1, ss, si, n, red);
+                const InnerSums s = parity_inner<W, KIND>(A, R, k1, ss, si, n, red, sc);
                 work += s.work + A.bs_work;
                 stats[4] += s.nu;
                 stats[5] += s.nn;
@@ -760,7 +769,9 @@ hipError_t launch_portfolio_parity(const PortfolioParityHost& H, hipStream_t s) 
             W = (v >= 8) ? 8 : (v >= 4) ? 4 : (v >= 2) ? 2 : 1;
         }
     }
-    const size_t lds = sizeof(double) * (2 * (size_t)H.pf.d + kParityRed + 2 * kMaxPhi * kMaxMoments);
+    // 16 B a stock and 256 B from some 1100 stocks on: 10224 stocks fill a block's 160 KB.
+    const bool general = !exact_only && H.pf.nopt[2] != 0;
+    const size_t lds = sizeof(double) * ((size_t)H.pf.d + lds_shared_doubles(general, H.pf.d) + 2 * kMaxPhi * kMaxMoments);
     switch (W) {
     case 8: hipLaunchKernelGGL((k_portfolio_parity<8, PAR_EXACT>), dim3(H.blocks), dim3(512), lds, s, A); break;
     case 4: hipLaunchKernelGGL((k_portfolio_parity<4, PAR_EXACT>), dim3(H.blocks), dim3(256), lds, s, A); break;
@@ -768,7 +779,7 @@ hipError_t launch_portfolio_parity(const PortfolioParityHost& H, hipStream_t s) 
     default:
         if (exact_only)
             hipLaunchKernelGGL((k_portfolio_parity<1, PAR_EXACT>), dim3(H.blocks), dim3(64), lds, s, A);
-        else if (H.pf.nopt[2] == 0)
+        else if (!general)
             hipLaunchKernelGGL((k_portfolio_parity<1, PAR_NO_UNBIASED>), dim3(H.blocks), dim3(64), lds, s, A);
         else
             hipLaunchKernelGGL((k_portfolio_parity<1, PAR_GENERAL>), dim3(H.blocks), dim3(64), lds, s, A);
