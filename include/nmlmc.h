@@ -287,7 +287,8 @@ uint32_t nmlmc_last_group_lanes(void);
  * problem in the current form over segments of 4, 8, 16, 32, 64 and 128 inner units
  * per lane and grids of 4, 8 and 16 blocks per CU, on outer samples set apart
  * for tuning (ids from 2^45), and keeps the fastest for later calls at level
- * ell.  Writes the choice and its kernel time (any pointer may be NULL).  The
+ * ell; small calls that run as one launch, a block an outer sample, do so
+ * whatever was tuned.  Writes the choice and its kernel time (any pointer may be NULL).  The
  * choices are dropped when a problem is staged or the adaptive rule changes;
  * per-sample results never depend on them. */
 int nmlmc_autotune_level(uint32_t ell, uint64_t M, uint32_t* segment, uint32_t* blocks_per_cu, double* ms);

@@ -923,7 +923,7 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
         const int few = general ? 20 : fp64 ? 22 : 18, many = general ? 22 : 24;
         sh.bpc = all < (1ull << few) ? 2 : all < (1ull << many) ? 4 : 8;
     }
-    bool chosen = t != tuned.end();
+    bool chosen = false;
     if (lanes_override) {
         sh.S = lanes_override;
         chosen = true;
@@ -963,8 +963,10 @@ bool Engine::residue_call(uint64_t M, ShapeKind kind, bool fp64, const BatchedCo
 //   level 5 (128) 1.5 times as long;
 // books, mixed: 2-3 times 10^3 at level 2 (16) 0.8 of the sequence, run 64 1.2 times as long; FP64: run 16
 //   equal, 32 1.2 times as long.
-// An explicit or tuned segment, and the sequence's own settings, ask for the
-// sequence; NMLMC_BLOCK_CALLS=0/1 for either where both can take the call.
+// An explicit segment, and the sequence's own settings, ask for the sequence; a tuned
+// one is the sequence's, which a call below these lines leaves all the same (1000 mixed
+// samples at level 3, tuned: 134 us as the sequence, 78 here).  NMLMC_BLOCK_CALLS=0/1 for
+// either where both can take the call.
 bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) {
     if (kind != ShapeKind::model && kind != ShapeKind::exact_book) return false;
     if (c.ell > 0 && !c.ep.antithetic) return false;
@@ -983,8 +985,8 @@ bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, con
 }
 
 // Times the batched level call (ell, M) of the staged problem in the current
-// form over candidate launch shapes and keeps the fastest for later calls at
-// this level: segments of 4, 8, 16, 32, 64 and 128 units at 8 blocks per CU,
+// form over candidate shapes of the launch sequence and keeps the fastest for later
+// calls at this level (those that block_call does not take): segments of 4, 8, 16, 32, 64 and 128 units at 8 blocks per CU,
 // then 4 and 16 blocks per CU at the best segment (the small segments spread
 // the few large draw groups of the high levels over more lanes; the large ones
 // pay fewer hand-offs at the low levels).  Each candidate runs twice (the
