@@ -218,6 +218,7 @@ int Engine::batch_sample(uint32_t ell, const uint64_t* Ms, sample_output* outs) 
     H.R_tau = pf_R;
     H.bs_work = 0.;
     H.mixed = form == NMLMC_FORM_MIXED;
+    for (const BatchInst& b : batch) H.mixed = H.mixed && b.pf.mix_units;
     H.exact_only = exact_only;
     H.multi = true;
     bool coupled = false;

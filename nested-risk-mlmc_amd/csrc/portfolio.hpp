@@ -26,7 +26,7 @@ struct StockRec {
 // data_ex (portfolio_sampler.cpp:94-132) with device pointers.
 // One Exact option for the FP32 inner loop of the mixed form (16 bytes).  Stock
 // levels and strikes are in units of the stock's S0, so that a stock needs four
-// constants (one load) and no division.
+// constants (one load) and no division (PortfolioDevice::mix_units: S0 is a unit).
 struct MixRec {
     float K;         // strike / S0
     float sTt;       // sqrt(T - tau)
@@ -109,6 +109,10 @@ struct PortfolioDevice {
     double compute_prob[3];
     uint32_t options_count;
     double prob_norm, total_std;
+    // 1: every Exact option's stock has S0 > 0 and a strike below 2^60 S0, so that levels
+    // and strikes over S0 are floats (a digital's payoff takes them times 2^60).  0: the
+    // mixed form runs the book's terms in FP64.
+    uint32_t mix_units;
 };
 
 // Device-side staging (stage.hip): builds the guides and the Exact records from

@@ -155,6 +155,7 @@ int Engine::stage_portfolio(const portfolio_data* data) {
     P.options_count = 0;
     double w_est0 = 0.;
     bool w_est_same = true;
+    P.mix_units = 1;
     for (int m = 0; m < 3; m++) {
         const option_params* ops = (const option_params*)data->options[m].data;
         double* cdf = (double*)(host + o_cdf[m]);
@@ -181,6 +182,10 @@ int Engine::stage_portfolio(const portfolio_data* data) {
             P.compute_prob[m] += o.prob;
             if (P.options_count == 0 && j == 0) w_est0 = o.W_est;
             w_est_same = w_est_same && o.W_est == w_est0;
+            if (m == 1) {
+                const double S0 = stocks[o.stock_ind].S0;
+                if (!(S0 > 0. && std::fabs(o.strike) < 0x1p60 * S0)) P.mix_units = 0;
+            }
         }
         if (n[m]) {
             std::memcpy(host + o_opt[m], ops, sizeof(OptionRec) * n[m]);
@@ -366,7 +371,7 @@ int Engine::sample_portfolio_batched(uint32_t ell, uint64_t M, uint64_t outer_of
     H.R_tau = pf_R;
     H.bs_work = pf_bs_work;
     H.blocks = (uint32_t)device_cus() * sh.bpc;
-    H.mixed = form == NMLMC_FORM_MIXED;
+    H.mixed = form == NMLMC_FORM_MIXED && pf.mix_units;
     H.multi = false;
     H.R32 = (H.mixed && H.exact_only) ? pf_R32 : nullptr;
     last_kernel = sh.block ? "k_b_block" : "k_b_final";
