@@ -874,7 +874,16 @@ uint64_t Engine::batched_chunk() {
 // pair of each; never fewer than 4 or 16 units and always 8 blocks were 15-28%
 // off, 60% for books with Unbiased options.
 // Model calls whose whole first group fits one lane take a segment of it (no pool
-// entries, no hand-offs: level 1 of the non-adaptive sweep 294 -> 183 us).  Coupled
+// entries, no hand-offs: level 1 of the non-adaptive sweep 294 -> 183 us).  Adaptive ones
+// from half a wave a SIMD on, 2^15 samples, or 3 2^14 where finals are long (FP64, us split /
+// whole: 50000 samples of 10 units, cap 2^2, 123 / 94, 200000 of them 255 / 153, of 5 units
+// 195 / 107, 131000 of 13 units, cap 2^4, 197 / 146; 33000 of those 116 / 124); 16 units
+// under a cap of 2^6 from 2^17 on, the line that a test of the segments holds (131000
+// samples 251 / 204).  From 2^16 on at least 8 units, 16 mixed: a refined sample's final then
+// fits as well (2 units, 131000 mixed samples, 4 / 8: 121 / 87 us; 4 units, 200000, 8 / 16: 129 /
+// 116).  A first group of 1024 units and more takes no fewer than 4 (reference model; FP64 shift
+// model 2): the finals are 2^cap as long, and how many are, `all` does not tell (30 samples of
+// 2048 units under a cap of 2^6, most of them refined to it, 1 / 4: 236 / 132 us).  Coupled
 // paths at few units are long and uneven: at most 2 (2^17 units: 480-720 us, with 4
 // 850-1400).
 //
@@ -909,9 +918,16 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
         for (uint32_t S : {32u, 64u})
             if (m * ((units + S - 1) / S) >= (1ull << 19)) sh.S = std::max(sh.S, S);
         if (kind == ShapeKind::model) {
-            const bool whole = adaptive ? units <= 16 && all >= (fp64 ? 1ull << 21 : 1ull << 18)
-                                        : units <= 16 || (units <= 32 && m >= 4096) || (units <= 64 && m >= 32768);
-            if (whole) sh.S = std::max(sh.S, pow2_ceil_u32(units));
+            if (adaptive) {
+                const bool long_finals = c.cf.max > 8 * c.cf.base;
+                const bool halves = fp64 && units == 16 && c.cf.max >= 64 * c.cf.base;
+                const uint64_t line = halves ? 1ull << 17 : long_finals ? 3ull << 14 : 1ull << 15;
+                if (units <= 16 && (m >= line || (!fp64 && all >= (1ull << 18))))
+                    sh.S = std::max({sh.S, m < (1ull << 16) ? 1u : fp64 ? 8u : 16u, pow2_ceil_u32(units)});
+                if (units >= 1024) sh.S = std::max(sh.S, spu == 1 ? 4u : fp64 ? 2u : 1u);
+            } else if (units <= 16 || (units <= 32 && m >= 4096) || (units <= 64 && m >= 32768)) {
+                sh.S = std::max(sh.S, pow2_ceil_u32(units));
+            }
         }
         if (kind == ShapeKind::coupled && all < (1ull << 18)) sh.S = std::min(sh.S, 2u);
         if (residues) {
@@ -955,19 +971,24 @@ bool Engine::residue_call(uint64_t M, ShapeKind kind, bool fp64, const BatchedCo
 // the launch sequence: few outer samples (each takes a block's set-up and sums,
 // the sequence's launches are shared by all) whose largest count is not a long run a
 // lane (the sequence splits a long sample over the chip).  `run`: units a lane of the
-// largest count.  Measured (block against sequence, us), lines where it still wins:
-// mixed model: 1000 samples at level 3 (run 32) 78 / 134, 3000 at level 4 (64) 114 / 152,
-//   1000 at level 5 (128) 124 / 158, 300 at level 5 (128) 61 / 137; beyond: 10000 at level 3 (2) 142 /
-//   99, 2000 at level 6 (256) equal, 1000 at level 8 (1024) 1.45 times as long;
-// FP64 model: 3000 at level 2 (16) 104 / 128, 300 at level 6 (256) 76 / 107; beyond: 1000 at
-//   level 5 (128) 1.5 times as long;
+// largest count.  How many samples run that long is not known before (it depends on the
+// threshold), so the lines hold for those of the reference model, of which many do.
+// Block time over the sequence's, 1 to 2000 samples, N0 from 32 to 3000, caps up to 2^6 and
+// not adaptive, both models:
+// mixed model: run 32 0.33-0.85, 64 0.37-0.95, 128 0.37-1.1, 256 and 100 samples 0.4-1.2 (300
+//   samples up to 2.0), 512 up to 3;
+// FP64 model: run 32 0.44-0.96, 64 0.46-1.35 (100 samples up to 1.15), 128 up to 1.8, 512 up to 4;
 // books, mixed: 2-3 times 10^3 at level 2 (16) 0.8 of the sequence, run 64 1.2 times as long; FP64: run 16
-//   equal, 32 1.2 times as long.
+//   equal, 32 1.2 times as long.  Without a correlation factor one lane draws an outer sample's
+//   stocks (some 1.2 us each, beside the other blocks of the CU): 1000 FP64 samples of 24 stocks
+//   84 us instead of 79, of 48 stocks 121 and 92; 2000, which take two turns of the blocks, of 2 stocks 67
+//   and 69, of 16 stocks 110 and 77, of 100 stocks 370 and 127.
+// 1000 mixed samples at level 3 (run 32) take 78 us instead of 134.
 // An explicit segment, and the sequence's own settings, ask for the sequence; a tuned
 // one is the sequence's, which a call below these lines leaves all the same (1000 mixed
 // samples at level 3, tuned: 134 us as the sequence, 78 here).  NMLMC_BLOCK_CALLS=0/1 for
 // either where both can take the call.
-bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) {
+bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) const {
     if (kind != ShapeKind::model && kind != ShapeKind::exact_book) return false;
     if (c.ell > 0 && !c.ep.antithetic) return false;
     if (c.cf.base % spu || c.cf.max % spu) return false;
@@ -978,10 +999,13 @@ bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, con
     if (const char* e = getenv("NMLMC_BLOCK_CALLS")) return e[0] != '0';
     if (c.redo_all || !fused_enabled() || getenv("NMLMC_FINAL_POOL") || getenv("NMLMC_TEST_SEGMENT_MIN")) return false;
     if (residue_call(M, kind, fp64, c)) return false;
-    const uint64_t run = (c.cf.max / spu + 255) / 256, base = (c.cf.base / spu + 255) / 256;
-    if (kind == ShapeKind::exact_book) return M <= 2048 && run <= (fp64 ? 8 : 16);
-    if (fp64) return (M <= 3072 && run <= 32) || (M <= 512 && run <= 256 && base <= 16);
-    return (M <= 3072 && run <= 64) || (M <= 1024 && run <= 128) || (M <= 512 && run <= 512);
+    const uint64_t run = (c.cf.max / spu + 255) / 256;
+    if (kind == ShapeKind::exact_book) {
+        const uint32_t serial = pf.chol ? 0 : pf.d;
+        return M <= (serial > 4 ? 1024 : 2048) && serial <= 24 && run <= (fp64 ? 8 : 16);
+    }
+    if (fp64) return (M <= 3072 && run <= 32) || (M <= 128 && run <= 64);
+    return (M <= 3072 && run <= 64) || (M <= 1024 && run <= 128) || (M <= 128 && run <= (spu == 1 ? 192 : 256));
 }
 
 // Times the batched level call (ell, M) of the staged problem in the current

@@ -150,7 +150,7 @@ struct Engine {
     // book on level-coupled paths.
     enum class ShapeKind { model, exact_book, general, coupled };
     static bool residue_call(uint64_t M, ShapeKind kind, bool fp64, const BatchedCommon& c);
-    static bool block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c);
+    bool block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) const;
     Shape batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
                         uint32_t lanes_override);
     int autotune_level(uint32_t ell, uint64_t M, Shape& best, double& best_ms);
