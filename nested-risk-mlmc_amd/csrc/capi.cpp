@@ -867,7 +867,9 @@ uint64_t Engine::batched_chunk() {
 // Segment.  Every lane walks its segments serially and every segment costs a
 // hand-off, so a call takes about a S + b all / S: the best S grows as the root
 // of `all`.  S is the power of two below sqrt(all / 2^k) (k: 14, or 15 or 16
-// where a unit costs more or no refinement follows), up to 16, or 32 for the mixed
+// where a unit costs more or no refinement follows; FP64 model groups of 17 to 32 units, whose
+// finals fit two or four segments of 16, 14: 100000 samples of 32 units, cap 2^2, 8 / 16 units
+// 340 / 293 us), up to 16, or 32 for the mixed
 // model's cheap units; from 2^19 segments of 32 or 64 units on, those.  Measured
 // over 280 calls (300 to 10^6 outer samples, levels 0 to 10, every form and
 // kind, S from 1 to 64 and 1 to 16 blocks a CU) the rule is 2-6% from the best
@@ -910,7 +912,7 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
         const uint64_t m = std::min(M, batched_chunk());
         const uint64_t all = m * units;
         int k = 14;
-        if (kind == ShapeKind::model && fp64) k = adaptive ? 16 : 15;
+        if (kind == ShapeKind::model && fp64) k = !adaptive ? 15 : units > 16 && units <= 32 ? 14 : 16;
         else if (kind == ShapeKind::exact_book) k = adaptive ? (fp64 ? 15 : 14) : 16;
         const uint32_t most = kind == ShapeKind::model && !fp64 ? 32 : 16;
         sh.S = 1;

@@ -77,11 +77,11 @@ def test_long_groups(nm, monkeypatch, form, variant, segment):
 
 
 @pytest.mark.parametrize("form, N0, cap, calls", [
-    ("batched", 20, 2, [(32767, 4), (32768, 16)]), ("batched", 20, 4, [(49151, 4), (49152, 16)]),
+    ("batched", 20, 2, [(32767, 4), (32768, 16)]), ("batched", 50, 2, [(41943, 8), (41944, 16)]), ("batched", 20, 4, [(49151, 4), (49152, 16)]),
     ("batched", 26, 6, [(49151, 4), (49152, 16)]), ("batched", 4, 2, [(65535, 2), (65536, 8)]),
     ("mixed", 4, 2, [(65535, 4), (65536, 16)]), ("mixed", 10, 2, [(32767, 4), (32768, 8)]),
 ])
-def test_whole_groups(nm, monkeypatch, form, N0, cap, calls):
+def test_segments_of_first_groups(nm, monkeypatch, form, N0, cap, calls):
     nm.init_nestedmc_sampler(1, N0, 2, 0.0, True)
     nm.set_adaptive_rule(1, cap)
     nm.set_form(nm.FORM_MIXED if form == "mixed" else nm.FORM_BATCHED)
