@@ -14,7 +14,7 @@ both forms are driven to RMSE eps by the MLMC driver (time to eps).
 
 roofline: a launch is one level call's kernel chain (k_b_zero, k_b_init, one
 k_b_test per refinement round, k_b_final_count/alloc/fill, k_b_final,
-k_b_redo_split, k_b_redo_seq), which is VALU-bound (integer Threefry + Box-Muller + compensated
+k_b_redo_split, k_b_redo_seq), which is VALU-bound (integer Threefry + Box-Muller + the
 sums; no input data, about 1 KB of queue and item-state traffic per outer
 sample), so achieved = algorithmic VALU lane-ops per launch (inner samples x ops
 per inner sample + outer samples x ops per outer sample, counts in
@@ -124,7 +124,7 @@ def autotune(nm, M0, levels):
 def ops_per_sample(form):
     with open(os.path.join(ROOT, "nested-risk-mlmc_amd", "opcount.json")) as f:
         oc = json.load(f)
-    key = "mixed" if form == 2 else "fp64"
+    key = ("plain", "fp64", "mixed")[form]
     return oc["shift_model"][key]["inner"], oc["shift_model"][key]["outer"]
 
 
