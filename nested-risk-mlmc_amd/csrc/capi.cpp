@@ -894,9 +894,9 @@ uint64_t Engine::batched_chunk() {
 // CU for few units (a call of 1000 mixed samples 174 -> 128 us), 4 up to 2^24, then
 // 8, which balance better (10^7 samples of the model, not adaptive: 1015 -> 915 us).
 //
-// Calls whose differences may be rounding residues (residue_call) keep the segment
-// that fixes those residues: the largest of 64, 32, 16 or 8 units that leaves 2^19
-// segments, else 16, or 4 from 1024 units on.
+// Calls whose differences may be rounding residues keep the segment that fixes those
+// (residue_segment): the largest of 64, 32, 16 or 8 units that leaves 2^19 segments, else
+// 16, or 4 from 1024 units on.
 Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
                                     uint32_t lanes_override) {
     if (force.S) return force;
@@ -905,7 +905,6 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
     if (t != tuned.end()) {
         sh = t->second;
     } else {
-        const bool residues = residue_call(M, kind, form != NMLMC_FORM_MIXED, c);
         const bool adaptive = c.cf.max > 2 * c.cf.base, fp64 = form != NMLMC_FORM_MIXED;
         const uint64_t group = adaptive ? c.cf.base : c.cf.max;
         const uint64_t units = (group + spu - 1) / spu;
@@ -932,11 +931,7 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
             }
         }
         if (kind == ShapeKind::coupled && all < (1ull << 18)) sh.S = std::min(sh.S, 2u);
-        if (residues) {
-            sh.S = units >= 1024 ? 4 : 16;
-            for (uint32_t S : {8u, 16u, 32u, 64u})
-                if (m * ((units + S - 1) / S) >= (1ull << 19)) sh.S = std::max(sh.S, S);
-        }
+        if (const uint32_t S = residue_segment(M, spu, kind, fp64, c)) sh.S = S;
         const bool general = kind == ShapeKind::general || kind == ShapeKind::coupled;
         const int few = general ? 20 : fp64 ? 22 : 18, many = general ? 22 : 24;
         sh.bpc = all < (1ull << few) ? 2 : all < (1ull << many) ? 4 : 8;
@@ -953,20 +948,31 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
     return sh;
 }
 
-// True for the FP64 model's antithetic levels with a loss that is no indicator and
-// fewer than 2^15 outer samples.  There phi_fine - phi_coarse of an outer sample whose
-// groups all lie on one side of the threshold is 0 but for the last places of its
-// means, and a call may hold no other kind (at level 8 some 250 outer samples, a
-// dozen above the threshold): its difference sums are then residues of the order in
-// which the inner samples were added, 10^-16 and of either sign.  The order is part
-// of such a call's results, so it does not follow the tuning of other calls: own
-// segments (batched_shape), the launch sequence and its Box-Muller pair
-// (boxmuller_f64_lib).  The non-adaptive sweep pays 110 us at its levels 6 to 8 (1954, 691 and
-// 245 outer samples), which k_b_block would take: 1180 us instead of 1070.
-// From 2^15 samples on, hundreds straddle the threshold at the levels that have so
-// many (2^15 at level 3: some 80), and their differences exceed residues 10^12 times.
-bool Engine::residue_call(uint64_t M, ShapeKind kind, bool fp64, const BatchedCommon& c) {
-    return kind == ShapeKind::model && fp64 && c.ell > 0 && c.ep.antithetic && c.phi_type != PHI_INDICATOR && M < (1ull << 15);
+// The segment of a call whose differences may be rounding residues, 0 for others.
+//
+// FP64 model, antithetic levels, a loss that is no indicator: phi_fine - phi_coarse of an
+// outer sample whose groups all lie on one side of the threshold is 0 but for the last
+// places of its means, and a call of few outer samples may hold no other kind.  Its
+// difference sums are then residues of the order in which the inner samples were added,
+// 10^-16 and of either sign.  As long as a group's segments lie in two waves (the sum of two
+// is the same in either order) that order is fixed, and part of the call's results: such
+// calls keep their segments, the launch sequence and its Box-Muller pair
+// (boxmuller_f64_lib) whatever other calls are tuned to.  With more waves the sequence's
+// atomics decide from run to run (100 runs of level 8's 245 outer samples gave their most
+// frequent sum 13 to 41 times); nothing is kept there, and k_b_block's order, two waves a group,
+// is the same in every run.  From 2^15 outer samples on dozens and more straddle the
+// threshold, whose differences are 10^12 times the residues.
+// Level 6 of the non-adaptive sweep (1954 outer samples) pays 30 us for it, of 1107.
+uint32_t Engine::residue_segment(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) {
+    if (kind != ShapeKind::model || !fp64 || c.ell == 0 || !c.ep.antithetic || c.phi_type == PHI_INDICATOR ||
+        M >= (1ull << 15))
+        return 0;
+    const uint64_t units = ((c.cf.max > 2 * c.cf.base ? c.cf.base : c.cf.max) + spu - 1) / spu;
+    uint32_t S = units >= 1024 ? 4 : 16;
+    for (uint32_t s : {8u, 16u, 32u, 64u})
+        if (M * ((units + s - 1) / s) >= (1ull << 19)) S = std::max(S, s);
+    const uint64_t group = (std::min(c.cf.base, c.cc.base) + spu - 1) / spu;
+    return group <= 128 * (uint64_t)S ? S : 0;
 }
 
 // True when a level call goes to k_b_block, a block an outer sample, rather than to
@@ -1000,7 +1006,7 @@ bool Engine::block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, con
     }
     if (const char* e = getenv("NMLMC_BLOCK_CALLS")) return e[0] != '0';
     if (c.redo_all || !fused_enabled() || getenv("NMLMC_FINAL_POOL") || getenv("NMLMC_TEST_SEGMENT_MIN")) return false;
-    if (residue_call(M, kind, fp64, c)) return false;
+    if (residue_segment(M, spu, kind, fp64, c)) return false;
     const uint64_t run = (c.cf.max / spu + 255) / 256;
     if (kind == ShapeKind::exact_book) {
         const uint32_t serial = pf.chol ? 0 : pf.d;

@@ -149,7 +149,7 @@ struct Engine {
     // of Exact options only, another book's or a sampler class's, or those of a
     // book on level-coupled paths.
     enum class ShapeKind { model, exact_book, general, coupled };
-    static bool residue_call(uint64_t M, ShapeKind kind, bool fp64, const BatchedCommon& c);
+    static uint32_t residue_segment(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c);
     bool block_call(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) const;
     Shape batched_shape(uint32_t ell, uint64_t M, uint64_t spu, ShapeKind kind, const BatchedCommon& c,
                         uint32_t lanes_override);

@@ -4,8 +4,9 @@ With phi = max and antithetic groups they are the last places of the means, set 
 the order in which the inner samples were added: part of the call's results, the
 same whatever segments and launches other calls take.  Held bit by bit to digests of
 phi_fine and phi_coarse (sha256, first 16 digits) and to the difference sums, at the
-levels whose groups take at most two waves (the sum of two is the same in either order;
-with more the waves' atomics decide, run by run).  Last: which calls the rule covers."""
+levels whose groups take at most two waves of the launch sequence (the sum of two is the
+same in either order; with more its atomics decide, run by run).  Beyond, small calls are
+one launch whose order is the same in every run.  Last: which calls the rule covers."""
 import hashlib
 
 import pytest
@@ -39,8 +40,19 @@ def test_bits(nm, ell, M, digest, diff):
     nm.set_form(nm.FORM_PLAIN)
 
 
+@pytest.mark.parametrize("ell, M", [(7, 691), (8, 245), (9, 87)])
+def test_same_in_every_run(nm, ell, M):
+    _setup(nm, nm.PHI_MAX)
+    runs = {(o["phi_f"].tobytes(), o["phi_c"].tobytes())
+            for o in (nm.sample(ell, M, outer_offset=7, trace=True) for _ in range(12))}
+    assert len(runs) == 1
+    nm.cleanup_nestedmc_sampler()
+    nm.set_form(nm.FORM_PLAIN)
+
+
 @pytest.mark.parametrize("phi, anti, ell, M, kernel, segment", [
-    ("max", True, 6, 1954, "k_b_final", 4), ("max", True, 8, 245, "k_b_final", 4),
+    ("max", True, 6, 1954, "k_b_final", 4), ("max", True, 6, 40, "k_b_final", 4),
+    ("max", True, 7, 691, "k_b_block", 8), ("max", True, 8, 245, "k_b_block", 8),  # more than two waves
     ("max", True, 5, 5525, "k_b_final", 16), ("max", True, 2, 32767, "k_b_final", 16),
     ("max", True, 2, 32768, "k_b_final", 64),          # hundreds straddle
     ("max", True, 0, 300, "k_b_block", 16),            # no differences
