@@ -141,8 +141,8 @@ __global__ __launch_bounds__(256) void k_b_init(typename P::Args A) {
 // new at least a factor 2 from cur is certain without the interval.  The
 // uncertain ones go to the FP64 recheck (k_b_test with RECHECK).  With both bounds
 // doubled, and the model's e1 the wider one of its finals, the rechecks took 11% of
-// an MLMC run on the small book; a run takes 60.5 instead of 62.4 ms, the large
-// book's sweep 7.0 instead of 7.15 ms.
+// an MLMC run on the small book; a run of one seed takes 60.5 instead of 62.4 ms (runs of
+// other seeds do other amounts of work), the large book's sweep 7.0 instead of 7.15 ms.
 template <class P, int RULE>
 __device__ __forceinline__ bool decision_uncertain(const BatchedCommon& c, const LevelCounts& lc, double start,
                                                    uint64_t cur, double s1, double s2, double sab, double smm) {

@@ -959,7 +959,7 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
 // calls keep their segments, the launch sequence and its Box-Muller pair
 // (boxmuller_f64_lib) whatever other calls are tuned to.  With more waves the sequence's
 // atomics decide from run to run (100 runs of level 8's 245 outer samples gave their most
-// frequent sum 13 to 41 times); nothing is kept there, and k_b_block's order, two waves a group,
+// frequent sum 11 to 41 times); nothing is kept there, and k_b_block's order, two waves a group,
 // is the same in every run.  From 2^15 outer samples on dozens and more straddle the
 // threshold, whose differences are 10^12 times the residues.
 // Level 6 of the non-adaptive sweep (1954 outer samples) pays 30 us for it, of 1107.

@@ -530,10 +530,10 @@ __device__ __forceinline__ InnerSums parity_inner(const PortfolioParityArgs& A, 
     return r;
 }
 
-// Waves per SIMD the kernels are compiled for: 2, which leaves the Exact-only
-// kernel's two samples a lane in registers (small book's plain sweep 8.4 ms; at 3,
-// 384 B of scratch a lane, 9.3 ms; at 4, 528 B, 10.0 ms) and the general one's window
-// nearly so (the reference main's mix 5.7 ms; at 3 6.7 ms).
+// Waves per SIMD the kernels are compiled for: 2.  The Exact-only kernel then keeps its two
+// samples a lane in 243 to 248 VGPRs with 96 B of scratch (small book's plain sweep 8.4 ms; at
+// 3, 384 B of scratch a lane, 9.3 ms; at 4, 528 B, 10.0 ms); the general one spills 387 VGPRs,
+// 704 B a lane, of its window (the reference main's mix 5.7 ms; at 3 6.7 ms).
 #ifndef NMLMC_PLAIN_EXACT_WAVES
 #define NMLMC_PLAIN_EXACT_WAVES 2
 #endif

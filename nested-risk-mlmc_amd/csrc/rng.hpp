@@ -171,11 +171,11 @@ __device__ __forceinline__ void boxmuller_f64(uint64_t u0, uint64_t u1, double& 
     y = c * r;
 }
 
-// The same pair through the device library's functions; it differs from the
-// one above by a last-place rounding in some of its values.  The model's batched FP64
-// form keeps it: its difference sums are, at the levels where no outer sample
-// straddles the threshold, nothing but rounding residues of means that are
-// equal, and with other roundings they are other residues.
+// The same pair through the device library's functions; it differs from the one above by
+// a last-place rounding in some of its values.  The model's batched FP64 form keeps it: the
+// differences of calls on which no outer sample straddles the threshold are nothing but
+// rounding residues of means that are equal, and with other roundings they are other
+// residues (Engine::residue_segment).
 __device__ __forceinline__ void boxmuller_f64_lib(uint64_t u0, uint64_t u1, double& x, double& y) {
     double s, c;
     sincos(3.1415926535897932 * uneg11_f64(u0), &s, &c);
