@@ -72,17 +72,21 @@ __device__ __forceinline__ double derv_from_stock_d(const OptionRec& o, double S
     return o.w * (St_T / S0) * exp(-r * o.maturity) * df;
 }
 
-// sample_inner_bs (453-468).
+// sample_inner_bs (453-468) from its operands.
+__device__ __forceinline__ double bs_value_d(int type, double strike, double maturity, double w, double start,
+                                             double S0, double sigma, double R, double r, double tau, bool delta_cv) {
+    const double finish = exp(-r * tau) * bs_price_d(type, R, strike, r, maturity - tau, sigma);
+    const double val = w * (start - finish);
+    const double cv = delta_cv ? ((R - S0) * (w * bs_delta_d(type, S0, strike, r, maturity, sigma))) : 0.;
+    return val + cv;
+}
 template <class RT>
 __device__ __forceinline__ double inner_bs_d(const PortfolioDevice& pf, const OptionRec& o, RT R_tau,
                                              double& work) {
     work += o.W_est;
-    const uint32_t si = o.stock_ind;
-    const StockRec st = pf.stocks[si];
-    const double finish = exp(-pf.r * pf.tau) * bs_price_d(o.type, R_tau[si], o.strike, pf.r, o.maturity - pf.tau, st.sigma);
-    const double val = o.w * (o.start - finish);
-    const double cv = pf.use_delta_cv ? ((R_tau[si] - st.S0) * (o.w * bs_delta_d(o.type, st.S0, o.strike, pf.r, o.maturity, st.sigma))) : 0.;
-    return val + cv;
+    const StockRec st = pf.stocks[o.stock_ind];
+    return bs_value_d(o.type, o.strike, o.maturity, o.w, o.start, st.S0, st.sigma, R_tau[o.stock_ind], pf.r, pf.tau,
+                      pf.use_delta_cv);
 }
 
 // e^x: x = k ln 2 + (f + fl), |f| <= ln(2) / 2 (Cody and Waite's reduction with its remainder
