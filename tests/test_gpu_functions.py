@@ -182,15 +182,18 @@ def test_mixed_sums_within_the_decision_bounds(probe, variant, tau, count):
 @pytest.mark.parametrize("anti", [True, False])
 @pytest.mark.parametrize("cv", [True, False])
 @pytest.mark.parametrize("tau", [1.0 / 52, 0.2])
-def test_mixed_exact_term_within_its_scale(probe, anti, cv, tau):
+@pytest.mark.parametrize("level", ["fp32", "fp64"])
+def test_mixed_exact_term_within_its_scale(probe, anti, cv, tau, level):
     """Vanillas and digitals near and far from the money, strikes within 2^-17 of the level
-    among them (the FP64 level of the draw itself, and both sides of the window)."""
+    among them (the FP64 level of the draw itself, and both sides of the window); outer levels
+    that FP32 holds, and any, which the FP32 term rounds first."""
     u0, u1 = _pairs()
     n = len(u0)
     rs = np.random.RandomState(17)
     S0, T = 10.0 ** rs.uniform(-3, 5, n), rs.uniform(0.25, 4, n)
     sigma = rs.uniform(0.05, 1, n) / np.sqrt(T)
-    R = np.exp(rs.normal(0, 0.3, n)).astype(np.float32).astype(np.float64)
+    R = np.exp(rs.normal(0, 0.3, n))
+    R = R.astype(np.float32).astype(np.float64) if level == "fp32" else R
     typ = rs.choice([1., -1., 2., -2.], n)
     x, y, _ = (v.astype(np.float64) for v in _reference(u0, u1))
     drift = 0.05 - sigma * sigma / 2
