@@ -962,7 +962,8 @@ Engine::Shape Engine::batched_shape(uint32_t ell, uint64_t M, uint64_t spu, Shap
 // frequent sum 11 to 41 times); nothing is kept there, and k_b_block's order, two waves a group,
 // is the same in every run.  From 2^15 outer samples on dozens and more straddle the
 // threshold, whose differences are 10^12 times the residues.
-// Level 6 of the non-adaptive sweep (1954 outer samples) pays 30 us for it, of 1107.
+// Level 6 of the non-adaptive sweep (1954 outer samples) pays 30 us for it, of 1107; 832
+// samples at level 3 under a cap of 2^2 take 90 us, as k_b_block 46.
 uint32_t Engine::residue_segment(uint64_t M, uint64_t spu, ShapeKind kind, bool fp64, const BatchedCommon& c) {
     if (kind != ShapeKind::model || !fp64 || c.ell == 0 || !c.ep.antithetic || c.phi_type == PHI_INDICATOR ||
         M >= (1ull << 15))
